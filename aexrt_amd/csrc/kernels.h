@@ -330,8 +330,8 @@ hipError_t launch_conv_int8_pg16(const ConvParams& p, hipStream_t stream);
 hipError_t launch_quant_fused_pg16(const void* x, bool f16, int N, int C, int HW, uint32_t* packed,
                                    uint32_t* amax, hipStream_t stream);
 
-// YOLO output0 postprocess (decode + filter, class-wise NMS, top-k) in one
-// block; element (channel ch, anchor a) of output0 at out[ch * ch_stride + a *
+// YOLO output0 postprocess (decode + filter, class-wise NMS, top-k) of one
+// image; element (channel ch, anchor a) of output0 at out[ch * ch_stride + a *
 // a_stride].  Writes count[0] = detections and dets[0 .. count) as x1, y1,
 // x2, y2, score, class.  1 <= max_candidates <= kYoloMaxCandidates.  With
 // levels, out is the raw Detect head (64 DFL bin logits, then class logits;

@@ -5,12 +5,12 @@
 //
 // The reference uses three dispatches and appends candidates with an atomic
 // counter, so their order (and which ones survive the max_candidates cap) is
-// whatever order its threads ran in.  Here one 1024-thread block does all of
-// it in LDS: anchors are scored in chunks of 1024, compacted with a block
-// scan in anchor order (one of the orders the reference can produce, and a
-// deterministic one), then every candidate is marked and ranked.  output0 is
-// small (84 x 2100 floats at 320x320) and read once; the pairwise NMS over
-// at most max_candidates boxes is the only quadratic step.
+// whatever order its threads ran in.  Here candidates are in anchor order (one
+// of the orders the reference can produce, and a deterministic one).  Two
+// launches share a workspace: one scores every anchor (post_score_kernel),
+// one compacts, marks and ranks the candidates (post_select_kernel).  Without
+// a workspace (launches recorded into a graph, more anchors than it holds) one
+// 1024-thread block does all of it in LDS (yolo_decode_nms_topk_kernel).
 //
 // Two decoders feed the same NMS and top-k:
 // * decoded output0 ([4 (+1 objectness) + classes][anchors]: cx, cy, w, h,
@@ -27,8 +27,14 @@
 // wins), a candidate passes unless score < conf.  exp is post_exp below (the
 // reference's comes from its shader compiler and driver), so that results
 // are reproducible bit for bit on the host.
+#include <algorithm>
+#include <map>
+#include <mutex>
+
 #include "common.h"
 #include "kernels.h"
+
+extern "C" hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus*) __attribute__((weak));
 
 namespace aexrt {
 
@@ -238,6 +244,344 @@ __global__ __launch_bounds__(kPostThreads) void yolo_decode_nms_topk_kernel(Post
     }
 }
 
+// ---- the same over the whole GPU --------------------------------------------------
+//
+// One block is bound by its CU: at 8400 anchors x 80 classes it took 440 us,
+// 317 us at 2100 anchors with 512 candidates (a sigmoid per class and anchor,
+// then count^2 steps of NMS and of ranking).  Spread over the CUs both parts
+// are a chain of a few memory round trips: 14.6 + 14.0 us, and 14.5 + 18.2 us.
+
+// Workspace of one postprocess: per anchor the box and (score, class), a bit
+// per anchor that passed, then per candidate its rank and whether it is kept.
+constexpr int kWsAnchors = 36864;  // up to 1280 x 1280 pixels (33600)
+struct PostWs {
+    float4 box[kWsAnchors];
+    float2 score[kWsAnchors];
+    uint64_t passed[kWsAnchors / 64];
+    uint32_t mark[kYoloMaxCandidates];
+    uint32_t blocks_done;
+    uint32_t unused[63];
+};
+
+constexpr int kScoreAnchors = 64;  // anchors of a score block, four threads each
+constexpr int kScoreChunk = 20;    // class scores in flight per thread (a quarter of 80)
+
+// LAST: channels last (the four threads of an anchor are neighbours and read
+// its row); otherwise channels first (a wave reads 64 neighbouring anchors of
+// one class).  Each thread takes a quarter of the classes, then one side of the
+// box of an anchor that passes.
+template <bool DFL, bool LAST>
+__global__ __launch_bounds__(4 * kScoreAnchors) void post_score_kernel(PostParams p, PostWs* ws, int vec) {
+#pragma clang fp contract(off)
+    __shared__ float l_best[4][kScoreAnchors];
+    __shared__ int l_cls[4][kScoreAnchors];
+    const int tid = threadIdx.x;
+    const int al = LAST ? tid >> 2 : tid & (kScoreAnchors - 1);
+    const int part = LAST ? tid & 3 : tid / kScoreAnchors;
+    const int a = blockIdx.x * kScoreAnchors + al;
+    const bool on = a < p.anchors;
+    if (blockIdx.x == 0 && tid == 0) ws->blocks_done = 0u;
+    const float* col = p.out + (int64_t)(on ? a : 0) * p.a_stride;
+    const int64_t cs = LAST ? 1 : p.ch_stride;
+    const float* sc = col + (DFL ? 4 * kDflBins : (p.has_obj ? 5 : 4)) * cs;
+    const float obj = !DFL && p.has_obj ? col[4 * cs] : 1.0f;
+    const int per = (p.classes + 3) / 4;
+    const int lo = min(part * per, p.classes), hi = min(lo + per, p.classes);
+    // this quarter's first largest value, and the largest of its others
+    float m = -__builtin_inff(), next = -__builtin_inff();
+    int cls = 0;
+    for (int c0 = lo; c0 < hi; c0 += kScoreChunk) {
+        float t[kScoreChunk];
+        if (LAST && vec) {
+#pragma unroll
+            for (int i = 0; i < kScoreChunk; i += 4)
+                *reinterpret_cast<float4*>(t + i) = *reinterpret_cast<const float4*>(sc + min(c0 + i, hi - 4));
+        } else {
+#pragma unroll
+            for (int i = 0; i < kScoreChunk; ++i) t[i] = sc[min(c0 + i, hi - 1) * cs];
+        }
+#pragma unroll
+        for (int i = 0; i < kScoreChunk; ++i) {
+            const float s = DFL ? t[i] : obj * t[i];
+            if (c0 + i < hi) {
+                next = fmaxf(next, fminf(m, s));
+                if (s > m) {
+                    m = s;
+                    cls = c0 + i;
+                }
+            }
+        }
+    }
+    float best = m;
+    if constexpr (DFL) {
+        // the largest logit has the largest sigmoid; one so close that rounding can bring its
+        // sigmoid level (up to 8 the sigmoid still grows by over 50 ulp in 0.01; beyond -88 it is
+        // 0 for all) has the sigmoids decide
+        const float near = m < -80.0f ? -__builtin_inff() : fminf(m, 8.0f) - 0.01f;
+        best = hi > lo ? post_sigmoid(m) : -__builtin_inff();
+        if (hi > lo && next >= near) {
+            best = -__builtin_inff();
+            for (int c = lo; c < hi; ++c) {
+                const float s = post_sigmoid(sc[c * cs]);
+                if (s > best) {
+                    best = s;
+                    cls = c;
+                }
+            }
+        }
+    }
+    if (part == 0) {
+        // the comparison starts at class 0: a NaN there stays
+        const float s0 = DFL ? sc[0] : obj * sc[0];
+        if (s0 != s0) {
+            best = s0;
+            cls = 0;
+        }
+    }
+    l_best[part][al] = best;
+    l_cls[part][al] = cls;
+    __syncthreads();
+    best = l_best[0][al];
+    cls = l_cls[0][al];
+#pragma unroll
+    for (int q = 1; q < 4; ++q) {
+        const float b = l_best[q][al];
+        if (b > best) {
+            best = b;
+            cls = l_cls[q][al];
+        }
+    }
+    const bool pass = on && !(best < p.conf);
+    if (pass) {
+        float coord;  // x1, y1, x2, y2
+        if constexpr (DFL) {
+            // side `part`: softmax expectation of its 16 bins
+            float v[kDflBins];
+#pragma unroll
+            for (int b = 0; b < kDflBins; ++b) v[b] = col[(part * kDflBins + b) * cs];
+            float top = -3.402823e38f;
+#pragma unroll
+            for (int b = 0; b < kDflBins; ++b) top = fmaxf(top, v[b]);
+            float sum = 0.0f, acc = 0.0f;
+#pragma unroll
+            for (int b = 0; b < kDflBins; ++b) {
+                const float e = post_exp(v[b] - top);
+                sum = sum + e;
+                acc = acc + e * (float)b;
+            }
+            const float dist = acc / fmaxf(sum, 1e-20f);
+            int l = 0;
+            while (l + 1 < p.nlev && a >= p.lev_off[l + 1]) ++l;
+            const int pos = a - p.lev_off[l];
+            const int gy = pos / p.lev_w[l];
+            const float ctr = (float)(part & 1 ? gy : pos - gy * p.lev_w[l]) + 0.5f;
+            coord = (part < 2 ? ctr - dist : ctr + dist) * p.lev_stride[l];
+        } else {
+            const float ctr = col[(part & 1) * cs], half = 0.5f * col[(2 + (part & 1)) * cs];
+            coord = part < 2 ? ctr - half : ctr + half;
+        }
+        reinterpret_cast<float*>(ws->box + a)[part] = coord;
+        if (part == 0) ws->score[a] = make_float2(best, (float)cls);
+    }
+    // the pass bits of the 64 anchors (a wave of channels first, 16 a wave otherwise)
+    if constexpr (LAST) {
+        uint64_t b = __ballot(pass && part == 0);
+        // every fourth bit -> 16 bits
+        b = (b | (b >> 3)) & 0x0303030303030303ull;
+        b = (b | (b >> 6)) & 0x000F000F000F000Full;
+        b = (b | (b >> 12)) & 0x000000FF000000FFull;
+        if ((tid & 63) == 0)
+            reinterpret_cast<uint16_t*>(ws->passed + blockIdx.x)[tid >> 6] = (uint16_t)(b | (b >> 24));
+    } else {
+        const uint64_t b = __ballot(pass);
+        if (tid == 0) ws->passed[blockIdx.x] = b;
+    }
+}
+
+// Total order of scores as unsigned keys: larger score, larger key; -0 counts as
+// 0 and a NaN comes first, so that ranks are a permutation.
+__device__ __forceinline__ uint32_t score_key(float s) {
+    if (s != s) return 0xFFFFFFFFu;
+    const uint32_t u = __float_as_uint(s + 0.0f);
+    return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+}
+
+constexpr int kSelThreads = 512;
+constexpr int kSelWaves = kSelThreads / 64;
+constexpr uint32_t kKept = 0x80000000u;
+
+// Sum of v over the threads before this one; total = the block's sum.  sums:
+// one word per wave.
+__device__ __forceinline__ uint32_t block_scan(uint32_t v, uint32_t* sums, uint32_t& total) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    uint32_t x = v;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t y = (uint32_t)__shfl_up((int)x, o, 64);
+        if (lane >= o) x += y;
+    }
+    __syncthreads();  // sums of an earlier scan are read
+    if (lane == 63) sums[wave] = x;
+    __syncthreads();
+    uint32_t before = 0, all = 0;
+#pragma unroll
+    for (int w = 0; w < kSelWaves; ++w) {
+        const uint32_t t = sums[w];
+        before += w < wave ? t : 0u;
+        all += t;
+    }
+    total = all;
+    return before + x - v;
+}
+
+// Every block gathers all candidates into LDS, marks and ranks its share of
+// them (several threads to a candidate), and the last block to finish writes
+// the detections.  The count^2 steps of 512 candidates, many of one class, are
+// 50 us of one CU.
+__global__ __launch_bounds__(kSelThreads) void post_select_kernel(PostParams p, PostWs* ws) {
+    extern __shared__ float l_cand[];  // [max_cand][6] in anchor order, then a key each
+    uint32_t* l_key = reinterpret_cast<uint32_t*>(l_cand + 6 * p.max_cand);
+    __shared__ uint32_t l_sums[kSelWaves];
+    __shared__ uint32_t l_last;
+    const int tid = threadIdx.x;
+    const int words = (p.anchors + 63) / 64;
+    uint32_t found = 0;
+    for (int w0 = 0; w0 < words && found < (uint32_t)p.max_cand; w0 += kSelThreads) {
+        uint64_t b = w0 + tid < words ? ws->passed[w0 + tid] : 0ull;
+        uint32_t all;
+        uint32_t k = found + block_scan((uint32_t)__popcll(b), l_sums, all);
+        // candidate k's anchor, in its class word until the gather
+        for (; b && k < (uint32_t)p.max_cand; b &= b - 1, ++k)
+            l_cand[6 * k + 5] = __int_as_float((w0 + tid) * 64 + __builtin_ctzll(b));
+        found += all;
+    }
+    const int count = (int)min(found, (uint32_t)p.max_cand);
+    __syncthreads();
+    for (int i = tid; i < count; i += kSelThreads) {
+        const int a = __float_as_int(l_cand[6 * i + 5]);
+        const float4 b = ws->box[a];
+        const float2 s = ws->score[a];
+        float* c = l_cand + 6 * i;
+        c[0] = b.x;
+        c[1] = b.y;
+        c[2] = b.z;
+        c[3] = b.w;
+        c[4] = s.x;
+        c[5] = s.y;
+        l_key[i] = score_key(s.x);
+    }
+    __syncthreads();
+    // ---- this block's candidates: blockIdx, blockIdx + grid, ... ----
+    const int mine = count > (int)blockIdx.x ? (count - 1 - (int)blockIdx.x) / (int)gridDim.x + 1 : 0;
+    int per = 1;  // threads to a candidate
+    while (per < 64 && 2 * per * mine <= kSelThreads) per <<= 1;
+    for (int m0 = 0; m0 < mine; m0 += kSelThreads / per) {
+        const int m = m0 + tid / per, share = tid & (per - 1);
+        uint32_t rank = 0;
+        bool drop = false;
+        const int i = blockIdx.x + m * gridDim.x;
+        if (m < mine) {
+            const float* ci = l_cand + 6 * i;
+            const uint32_t ki = l_key[i];
+            const bool ordered = ci[4] == ci[4];  // a NaN score drops nothing and is not dropped
+            for (int j = share; j < count; j += per) {
+                const uint32_t kj = l_key[j];
+                if (!(kj > ki || (kj == ki && j < i))) continue;
+                ++rank;
+                const float* cj = l_cand + 6 * j;
+                if (!drop && ordered && cj[5] == ci[5] && cj[4] == cj[4]) drop = box_iou(ci, cj) > p.iou;
+            }
+        }
+        for (int o = 1; o < per; o <<= 1) {
+            rank += (uint32_t)__shfl_xor((int)rank, o, 64);
+            drop = __shfl_xor((int)drop, o, 64) || drop;
+        }
+        if (m < mine && share == 0)
+            __hip_atomic_store(&ws->mark[i], rank | (drop ? 0u : kKept), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    // ---- the last block: kept candidates in rank order ----
+    __threadfence();
+    __syncthreads();
+    if (tid == 0) l_last = atomicAdd(&ws->blocks_done, 1u) == gridDim.x - 1 ? 1u : 0u;
+    __syncthreads();
+    if (!l_last) return;
+    __threadfence();
+    uint32_t* l_by = l_key;  // by rank: candidate + 1, 0 when dropped
+    for (int i = tid; i < count; i += kSelThreads) {
+        const uint32_t mi = __hip_atomic_load(&ws->mark[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        l_by[mi & ~kKept] = mi & kKept ? (uint32_t)i + 1u : 0u;
+    }
+    __syncthreads();
+    uint32_t kept = 0;
+    for (int r0 = 0; r0 < count; r0 += kSelThreads) {
+        const uint32_t c = r0 + tid < count ? l_by[r0 + tid] : 0u;
+        uint32_t all;
+        const uint32_t row = kept + block_scan(c ? 1u : 0u, l_sums, all);
+        if (c && row < (uint32_t)p.max_det)
+            for (int k = 0; k < 6; ++k) p.dets[6 * (int64_t)row + k] = l_cand[6 * (c - 1) + k];
+        kept += all;
+    }
+    if (tid == 0) p.count[0] = min(kept, (uint32_t)p.max_det);
+}
+
+// Workspaces: a few per device, each handed from call to call in the order of
+// the streams (a call waits for the event behind the slot's last one), so that
+// calls on any number of threads and streams are safe.
+constexpr int kWsSlots = 4;
+__device__ PostWs g_post_ws[kWsSlots];
+
+struct WsPool {
+    PostWs* ws = nullptr;
+    hipEvent_t done[kWsSlots] = {};
+    hipStream_t last[kWsSlots] = {};
+    int next = 0;
+};
+std::mutex g_ws_mutex;
+std::map<int, WsPool> g_ws;
+
+// The device's pool, nullptr when it cannot be set up.
+WsPool* ws_pool() {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return nullptr;
+    WsPool& w = g_ws[dev];
+    if (!w.ws) {
+        for (hipEvent_t& e : w.done)
+            if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming | hipEventDisableSystemFence) != hipSuccess) {
+                e = nullptr;
+                return nullptr;
+            }
+        void* p = nullptr;
+        if (hipGetSymbolAddress(&p, HIP_SYMBOL(g_post_ws)) != hipSuccess) return nullptr;
+        w.ws = static_cast<PostWs*>(p);
+    }
+    return &w;
+}
+
+// A launch recorded into a graph may be replayed at any time, beside any other
+// call: it has no slot.
+bool recording(hipStream_t stream) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    // absent from the host stand-in of the HIP runtime, which records nothing here
+    if (!hipStreamIsCapturing) return false;
+    return hipStreamIsCapturing(stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
+}
+
+template <bool DFL>
+void launch_post(const PostParams& p, PostWs* ws, hipStream_t stream) {
+    const dim3 blocks((unsigned)((p.anchors + kScoreAnchors - 1) / kScoreAnchors));
+    const int cls_off = DFL ? 4 * kDflBins : (p.has_obj ? 5 : 4);
+    const int vec = p.a_stride % 4 == 0 && cls_off % 4 == 0 && p.classes % 16 == 0 &&
+                    reinterpret_cast<uintptr_t>(p.out) % 16 == 0;
+    if (p.ch_stride == 1)
+        hipLaunchKernelGGL((post_score_kernel<DFL, true>), blocks, dim3(4 * kScoreAnchors), 0, stream, p, ws, vec);
+    else
+        hipLaunchKernelGGL((post_score_kernel<DFL, false>), blocks, dim3(4 * kScoreAnchors), 0, stream, p, ws, vec);
+    // 16 candidates to a block: 32 threads to each
+    const int sel = std::min(64, (p.max_cand + 15) / 16);
+    hipLaunchKernelGGL(post_select_kernel, dim3((unsigned)sel), dim3(kSelThreads),
+                       (size_t)p.max_cand * 7 * sizeof(float), stream, p, ws);
+}
+
 }  // namespace
 
 hipError_t launch_yolo_decode_nms_topk(const float* out, int ch_stride, int a_stride, int anchors, int classes,
@@ -274,6 +618,26 @@ hipError_t launch_yolo_decode_nms_topk(const float* out, int ch_stride, int a_st
         p.lev_off[levels->n] = off;
         p.nlev = levels->n;
         if (off != anchors) return hipErrorInvalidValue;
+    }
+    if (anchors > 0 && anchors <= kWsAnchors && classes > 0 && !recording(stream)) {
+        std::lock_guard<std::mutex> lock(g_ws_mutex);
+        if (WsPool* w = ws_pool()) {
+            int slot = 0;  // this stream's, else the next in turn
+            while (slot < kWsSlots && w->last[slot] != stream) ++slot;
+            if (slot == kWsSlots) {
+                slot = w->next;
+                w->next = (w->next + 1) % kWsSlots;
+            }
+            // an event never recorded is complete
+            hipError_t e = hipStreamWaitEvent(stream, w->done[slot], 0);
+            if (e != hipSuccess) return e;
+            w->last[slot] = stream;
+            if (levels) launch_post<true>(p, w->ws + slot, stream);
+            else launch_post<false>(p, w->ws + slot, stream);
+            e = hipGetLastError();
+            const hipError_t r = hipEventRecord(w->done[slot], stream);
+            return e != hipSuccess ? e : r;
+        }
     }
     const size_t lds = (size_t)max_candidates * 7 * sizeof(float);
     if (levels)
