@@ -6,14 +6,16 @@
 //     per (position, 4 channels) scales computed in the conv;
 //   * plan flag 16 (AEXRT_HIP_CONV_INT8_PG16): the reference's strip amax of
 //     the input (RT:3219-3259) into scratch, then the pg16 conv;
-//   * otherwise: the per-tensor amax of the input (16-channel slots, striped)
-//     into scratch, then the prequantized conv that quantizes on load.
-// The scratch is the amax words: stripes x C/16 uint32, cleared by a fill
-// kernel before every use.  The library allocates it once per device and
+//   * otherwise: the per-tensor amax of the input, in parts, into scratch, then
+//     the prequantized conv that quantizes on load.
+// The scratch is the amax words: one per part of the input (each written by its
+// block, nothing to clear), or the strips' C/16 words, cleared by a fill kernel
+// before every use.  The library allocates it once per device and
 // keeps it for the process; calls that overlap on one device share it and
 // race.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <vector>
@@ -24,7 +26,10 @@ namespace aexrt {
 
 namespace {
 
-constexpr uint32_t kCmdStripes = 16;  // slot copies the amax pass spreads its atomics over
+// Parts of the amax pass: two blocks a CU, and no more words than a conv reads
+// (its waves read them all at their start).
+constexpr uint32_t kAmaxParts = 512;
+constexpr uint32_t kMaxGroups = 32;  // 16-channel groups a per-tensor command takes (512 channels)
 
 struct DeviceScratch {
     uint32_t* words = nullptr;
@@ -53,7 +58,9 @@ uint32_t* library_scratch(uint64_t words) {
 
 }  // namespace
 
-uint64_t int8_command_scratch_words(uint32_t in_channels) { return uint64_t(kCmdStripes) * ((in_channels + 15) / 16); }
+uint64_t int8_command_scratch_words(uint32_t in_channels) {
+    return std::max<uint64_t>(kAmaxParts, (in_channels + 15) / 16);
+}
 
 bool run_int8_command(const AexrtConv2DDesc& d, uint32_t algorithm, uint32_t flags, const AexrtHipTensorView& x,
                       const void* weight, const float* w_scale, const float* bias, const AexrtHipTensorView* residual,
@@ -85,26 +92,36 @@ bool run_int8_command(const AexrtConv2DDesc& d, uint32_t algorithm, uint32_t fla
         return launch_conv(p, algorithm, stream);
     }
     const bool pg16 = (flags & AEXRT_HIP_CONV_INT8_PG16) != 0;
-    const uint32_t stripes = pg16 ? 1u : kCmdStripes;
-    if (!scratch || scratch_words < uint64_t(stripes) * groups) {
+    if (!scratch || scratch_words < (pg16 ? groups : kAmaxParts)) {
         set_error("conv2d_int8: scratch smaller than the input's amax words");
         return false;
     }
+    if (!pg16 && groups > kMaxGroups) {
+        set_error("conv2d_int8: per-tensor commands take at most 512 input channels");
+        return false;
+    }
     xv.amax_slots = scratch;
-    xv.amax_stripes = stripes;
-    xv.amax_stripe_stride = stripes > 1 ? groups : 0;
     if (!build_conv_params(d, algorithm, flags, xv, weight, w_scale, bias, residual, y, nullptr, p, why)) {
         set_error("conv2d_int8: " + why);
         return false;
     }
     const __half* xd = static_cast<const __half*>(x.data);
     const int N = (int)d.batch, HW = (int)(d.in_h * d.in_w), C = (int)d.in_channels;
-    if (!check_hip(launch_fill_u32(scratch, uint64_t(stripes) * groups, 0u, stream), "conv2d_int8: clear amax"))
-        return false;
-    const hipError_t e = pg16 ? launch_amax_strips_nhwc(xd, x.n_stride, x.c_stride, N, HW, C, scratch, stream)
-                              : launch_amax_slots_nhwc(xd, x.n_stride, x.c_stride, N, HW, C,
-                                                       SlotRef{scratch, stripes, groups}, stream);
-    if (!check_hip(e, "conv2d_int8: amax pass")) return false;
+    if (pg16) {
+        if (!check_hip(launch_fill_u32(scratch, groups, 0u, stream), "conv2d_int8: clear amax") ||
+            !check_hip(launch_amax_strips_nhwc(xd, x.n_stride, x.c_stride, N, HW, C, scratch, stream),
+                       "conv2d_int8: amax pass"))
+            return false;
+    } else {
+        int parts = 0;
+        if (!check_hip(launch_amax_parts_nhwc(xd, x.n_stride, x.c_stride, N, HW, C, scratch, (int)kAmaxParts, &parts,
+                                              stream),
+                       "conv2d_int8: amax pass"))
+            return false;
+        // the conv takes the maximum over copies of one group
+        p.x_slots = SlotRef{scratch, (uint32_t)parts, 1u};
+        p.x_nslots = 1;
+    }
     return launch_conv(p, algorithm, stream);
 }
 
@@ -115,11 +132,11 @@ bool run_int8_command(const AexrtConv2DDesc& d, uint32_t algorithm, uint32_t fla
 // capture, tight serving loops, harnesses that forbid hipMalloc): the amax
 // words live in this file-scope array instead of library-allocated memory.
 // Each device holds its own copy until the process ends.  It covers convs of
-// up to kNoAllocMaxChannels input channels (16 stripes x C/16 words).
+// up to kNoAllocMaxChannels input channels.
 namespace aexrt {
 namespace {
 constexpr uint32_t kNoAllocMaxChannels = 4096;
-constexpr uint64_t kNoAllocWords = uint64_t(kCmdStripes) * (kNoAllocMaxChannels / 16);  // 16 KiB
+constexpr uint64_t kNoAllocWords = 4096;  // 16 KiB
 }  // namespace
 }  // namespace aexrt
 

@@ -302,6 +302,11 @@ hipError_t launch_winograd_f2x2(const ConvParams& p, hipStream_t stream);
 // (atomicMax, caller clears).  C % 16 == 0.
 hipError_t launch_amax_slots_nhwc(const __half* x, int64_t nstride, int32_t cstride, int N, int HW,
                                   int C, SlotRef slots, hipStream_t stream);
+// Per-tensor amax of an NHWC fp16 view in parts: parts[0 .. *count) hold the
+// maxima of as many shares of the tensor (*count <= max_parts, a host choice);
+// nothing to clear.  C % 16 == 0.
+hipError_t launch_amax_parts_nhwc(const __half* x, int64_t nstride, int32_t cstride, int N, int HW, int C,
+                                  uint32_t* parts, int max_parts, int* count, hipStream_t stream);
 // Strips of the reference's amax buffer over an NHWC fp16 view: max|x| of
 // image n, group g folded into slots[(n * C/16 + g) / N], i.e. memory strip
 // (n*C + 16g) / (16N) of the NCHW layout (slots[s] = the reference's

@@ -292,9 +292,9 @@ int aexrt_hip_conv2d_f32(const AexrtConv2DDesc* desc, uint32_t flags, const floa
  *     (RT:3314-3346, 4614-4762) quantizing on load.
  * algorithm 51/52/53; flags SILU / RESIDUAL / OUT_F32 / INT8_PG16; in_channels
  * % 16 == 0.  The amax words live in a scratch buffer the library allocates
- * on the current device at first use (16 x C/16 uint32, grown when a conv
- * needs more) and keeps until the process ends; every call clears what it
- * uses first.  Calls that overlap on one device share that scratch and race. */
+ * on the current device at first use (512 uint32, grown when a conv
+ * needs more) and keeps until the process ends; every call writes what it
+ * reads first.  Calls that overlap on one device share that scratch and race. */
 int aexrt_hip_conv2d_int8(const AexrtConv2DDesc* desc, uint32_t algorithm, uint32_t flags, const AexrtHipTensorView* x,
                           const void* weight, const float* w_scale, const float* bias,
                           const AexrtHipTensorView* residual, const AexrtHipTensorView* y, void* stream);
