@@ -81,6 +81,10 @@ bool tile_instantiated(const ConvTile& t) {
 }
 }  // namespace
 
+namespace {
+bool tile_forced() { return g_tile_override.load(std::memory_order_relaxed) != 0; }
+}  // namespace
+
 bool set_conv_tile_override(int jn, int pw, int ksw) {
     if (jn == 0 && pw == 0 && ksw == 0) {
         g_tile_override.store(0);
@@ -253,6 +257,12 @@ hipError_t launch_conv_igemm(const ConvParams& p0, bool int8, hipStream_t stream
             ConvChoice forced;
             if (forced_s1x1_choice(forced)) {
                 p.choice = forced;  // a forced tile that does not fit is an error
+                e = launch_conv_s1x1(p, int8, epi, stream);
+                if (e != hipSuccess) return e;
+                continue;
+            }
+            // no tile forced on the implicit GEMM either: the streaming kernel by its rule
+            if (!tile_forced() && choose_s1x1(p, int8, p.choice)) {
                 e = launch_conv_s1x1(p, int8, epi, stream);
                 if (e != hipSuccess) return e;
                 continue;

@@ -117,6 +117,39 @@ bool forced_s1x1_choice(ConvChoice& c) {
     return true;
 }
 
+// The tile of a conv without a measured choice, false when the implicit GEMM is
+// to run it.  One position subtile a wave on a persistent grid, and the most
+// channels per block (the input is loaded and quantized once per channel tile)
+// that still leave 192 tiles to spread over the CUs.  Over 90 shapes of 4 to 160
+// pixels a side, 16 to 512 channels and 1 to 64 images this is 3 % from the best
+// tile of either kernel (geometric mean; the implicit GEMM's choice 41 %), e.g.
+// 128 -> 256 at 40 x 40 4.8 us (6.3), 48 -> 48 at 80 x 80 x 32 13.0 (16.4).  Past
+// 256 channels a thread holds more than four input pieces of a tile and the tile
+// buffers soon leave room for one block a CU, whose quantizing and storing then
+// alternate with nothing beside them: with more than 640 tiles the implicit GEMM
+// is the faster one (400 -> 128 at 40 x 40 x 32: 20.3 against 22.3 us), below not
+// (384 -> 128 at 20 x 20 x 64: 13.2 against 10.8).
+bool choose_s1x1(const ConvParams& p, bool int8, ConvChoice& c) {
+    if (!s1x1_shape_ok(p, int8) || p.yup || p.xup) return false;
+    const int ocj = p.OCp / 16;
+    const int64_t nt = ((int64_t)p.M + 63) / 64;
+    int jq = 1;
+    while (jq < 8 && jq < ocj) jq <<= 1;
+    S1x1Params h{};
+    h.c = p;
+    auto fits = [&](int j) {
+        S1x1Tile t{j, 1, 0};
+        return s1x1_geometry(h, t);
+    };
+    while (jq > 1 && (nt * ((ocj + jq - 1) / jq) < 192 || !fits(jq))) jq >>= 1;
+    if (!fits(jq) || (p.C > 256 && nt * ((ocj + jq - 1) / jq) > 640)) return false;
+    c = ConvChoice{};
+    c.kind = 6;
+    c.jn = jq;
+    c.pw = 1;
+    return true;
+}
+
 int enumerate_s1x1_choices(const ConvParams& p, bool int8, ConvChoice* out, int cap) {
     // the launcher sets p.lin per batch slice; the strides decide it
     ConvParams q = p;

@@ -239,6 +239,8 @@ hipError_t launch_conv_s1x1(const ConvParams& p, bool int8, int epi, hipStream_t
 // streaming tile (on = false: off).  False for a tile without an instance.
 bool set_conv1x1_stream(int mode, int jq, int pq);  // 0 off, 1 persistent, 2 one tile per block
 bool forced_s1x1_choice(ConvChoice& c);
+// The streaming tile of a conv without a measured choice; false: the implicit GEMM.
+bool choose_s1x1(const ConvParams& p, bool int8, ConvChoice& c);
 // Band kernel of the network's first conv (3x3 pad 1, stride 1/2, fp32 NCHW
 // input of at most 3 channels read directly, fp16 SiLU output, OCp <= 64,
 // W % 4 == 0): whole output rows per tile, one fp16 MFMA per 16 positions and
