@@ -557,21 +557,51 @@ __global__ __launch_bounds__(kThreads) void nchw_f32_to_nhwc8_kernel(const float
     }
 }
 
-template <typename T>
-__global__ __launch_bounds__(kThreads) void nhwc_to_nchw_f32_kernel(const T* x, int64_t x_nstride,
-                                                                   int32_t x_cstride, float* y, int C,
-                                                                   int HW, int64_t total) {
-    const int64_t step = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += step) {
-        const int64_t pos = i % HW;
-        const int64_t t = i / HW;
-        const int c = (int)(t % C);
-        const int64_t n = t / C;
-        const int64_t src = n * x_nstride + pos * x_cstride + c;
-        float v;
-        if constexpr (sizeof(T) == 2) v = __half2float(reinterpret_cast<const __half*>(x)[src]);
-        else v = reinterpret_cast<const float*>(x)[src];
-        y[i] = v;
+// NHWC view -> dense fp32 NCHW through an LDS tile of 64 positions x tc (at most
+// 64) channels: reads run along the channels (VEC: 16 bytes a lane, where the
+// view's alignment and strides allow), writes along the positions, so both sides
+// move whole cache lines.  Bound by HBM: 64 x 2100 x 144 fp32 in 36 us, 4.3 TB/s
+// (129 us with a thread per output element, whose reads take a line each).
+constexpr int kTransPos = 64;
+
+template <typename T, bool VEC>
+__global__ __launch_bounds__(kThreads) void nhwc_to_nchw_f32_kernel(const T* x, int64_t x_nstride, int32_t x_cstride,
+                                                                   float* y, int C, int HW, int tc, int ctiles,
+                                                                   int ptiles, int64_t tiles, FastDiv fd_row) {
+    constexpr int E = VEC ? 16 / (int)sizeof(T) : 1;
+    __shared__ float t[64][kTransPos + 1];
+    const int row = tc / E;  // loads of one position
+    for (int64_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+        const int64_t np = tile / ctiles;
+        const int c0 = (int)(tile - np * ctiles) * tc;
+        const int64_t n = np / ptiles;
+        const int p0 = (int)(np - n * ptiles) * kTransPos;
+        const int nc = min(tc, C - c0), npos = min(kTransPos, HW - p0);
+        const T* xb = x + n * x_nstride + (int64_t)p0 * x_cstride + c0;
+        for (int i = threadIdx.x; i < npos * row; i += kThreads) {
+            const int pos = (int)fdiv((uint32_t)i, fd_row), c = (i - pos * row) * E;
+            if (c >= nc) continue;
+            const T* src = xb + (int64_t)pos * x_cstride + c;
+            if constexpr (VEC) {
+                const uint4 v = *reinterpret_cast<const uint4*>(src);
+                T e[E];
+                __builtin_memcpy(e, &v, 16);
+#pragma unroll
+                for (int k = 0; k < E; ++k) {
+                    if constexpr (sizeof(T) == 2) t[c + k][pos] = __half2float(e[k]);
+                    else t[c + k][pos] = e[k];
+                }
+            } else {
+                if constexpr (sizeof(T) == 2) t[c][pos] = __half2float(*src);
+                else t[c][pos] = *src;
+            }
+        }
+        __syncthreads();
+        const int pos = threadIdx.x & 63;
+        float* yb = y + (n * C + c0) * HW + p0 + pos;
+        if (pos < npos)
+            for (int c = threadIdx.x >> 6; c < nc; c += kThreads / 64) yb[(int64_t)c * HW] = t[c][pos];
+        __syncthreads();
     }
 }
 
@@ -749,16 +779,32 @@ hipError_t launch_nchw_f32_to_nhwc8(const float* x, __half* y, int N, int C, int
     return hipGetLastError();
 }
 
+namespace {
+template <typename T>
+hipError_t launch_to_nchw(const T* x, int64_t x_nstride, int32_t x_cstride, float* y, int N, int C, int HW,
+                          hipStream_t stream) {
+    if (N < 1 || C < 1 || HW < 1) return hipSuccess;
+    constexpr int E = 16 / (int)sizeof(T);
+    const bool vec = C % E == 0 && x_cstride % E == 0 && x_nstride % E == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0;
+    const int ctiles = (C + 63) / 64;
+    const int tc = ((C + ctiles - 1) / ctiles + 7) & ~7;
+    const int ptiles = (HW + kTransPos - 1) / kTransPos;
+    const int64_t tiles = (int64_t)N * ptiles * ctiles;
+    const dim3 grid((unsigned)std::min<int64_t>(tiles, 1 << 20));
+    if (vec)
+        hipLaunchKernelGGL((nhwc_to_nchw_f32_kernel<T, true>), grid, dim3(kThreads), 0, stream, x, x_nstride, x_cstride,
+                           y, C, HW, tc, ctiles, ptiles, tiles, make_fastdiv((uint32_t)(tc / E)));
+    else
+        hipLaunchKernelGGL((nhwc_to_nchw_f32_kernel<T, false>), grid, dim3(kThreads), 0, stream, x, x_nstride,
+                           x_cstride, y, C, HW, tc, ctiles, ptiles, tiles, make_fastdiv((uint32_t)tc));
+    return hipGetLastError();
+}
+}  // namespace
+
 hipError_t launch_nhwc_to_nchw_f32(const void* x, bool f16, int64_t x_nstride, int32_t x_cstride, float* y,
                                    int N, int C, int HW, hipStream_t stream) {
-    const int64_t total = (int64_t)N * C * HW;
-    if (f16)
-        hipLaunchKernelGGL(nhwc_to_nchw_f32_kernel<__half>, dim3(grid_for(total)), dim3(kThreads), 0, stream,
-                           reinterpret_cast<const __half*>(x), x_nstride, x_cstride, y, C, HW, total);
-    else
-        hipLaunchKernelGGL(nhwc_to_nchw_f32_kernel<float>, dim3(grid_for(total)), dim3(kThreads), 0, stream,
-                           reinterpret_cast<const float*>(x), x_nstride, x_cstride, y, C, HW, total);
-    return hipGetLastError();
+    return f16 ? launch_to_nchw(static_cast<const __half*>(x), x_nstride, x_cstride, y, N, C, HW, stream)
+               : launch_to_nchw(static_cast<const float*>(x), x_nstride, x_cstride, y, N, C, HW, stream);
 }
 
 }  // namespace aexrt
