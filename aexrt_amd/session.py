@@ -15,7 +15,7 @@ from typing import Any, Dict, Optional
 
 import numpy as np
 
-from .graph import Graph
+from .graph import Graph, infer_value_specs
 
 
 @dataclass(frozen=True)
@@ -53,6 +53,7 @@ class HipBackend(Backend):
         self.model = None
         self.engine_bytes: Optional[bytes] = None
         self.graph: Optional[Graph] = None
+        self.output_shape: Optional[tuple] = None
 
     def info(self) -> BackendInfo:
         caps = self.model.capabilities if self.model is not None else {}
@@ -72,18 +73,13 @@ class HipBackend(Backend):
             algo = E.w8a8_algo_map(replay, names)
         self.engine_bytes = E.build_aexrt_engine(graph, precision=self.precision, algo_overrides=algo)
         self.model = NativeHipYoloModel(self.engine_bytes, self.device_index)
+        self.output_shape = infer_value_specs(graph)[graph.outputs[0]].shape
 
     def run(self, inputs: Dict[str, Any]) -> Dict[str, Any]:
         (name, x), = inputs.items()
         self.model.run(np.asarray(x, dtype=np.float32))
         out = self.model.output()
-        spec_shape = self._output_shape()
-        return {self.graph.outputs[0]: out.reshape(spec_shape)}
-
-    def _output_shape(self):
-        from .graph import infer_value_specs
-
-        return infer_value_specs(self.graph)[self.graph.outputs[0]].shape
+        return {self.graph.outputs[0]: out.reshape(self.output_shape)}
 
 
 class InferenceSession:
