@@ -5,11 +5,11 @@
 // (RT:2533-2548), the 16 transform points become 16 independent GEMMs
 // M_r[tile][oc] = sum_c V_r[tile][c] * U_r[c][oc] with U = G g G^T prepared
 // by the compiler (packed layout 3), and the output is A^T M A + bias
-// (RT:2612-2619).  A block owns 32 tiles x 32 output channels; each wave
-// computes the same 16x16 (tile, oc) sub-block for all 16 points, so after
-// the K loop every lane holds all 16 points of its (tile, oc) pairs and the
-// output transform runs in registers.  V is staged in LDS per 32-channel
-// chunk; U ([16][OCp][Cp] fp16, repacked at load) streams from L2.
+// (RT:2612-2619).  A block owns 16 or 32 tiles x 32 or 64 output channels; its V
+// is staged in LDS per channel chunk, U ([16][OCp][Cp] fp16, repacked at load)
+// streams from L2, and the output transform runs in registers.
+#include <algorithm>
+
 #include "common.h"
 #include "kernels.h"
 
@@ -17,10 +17,9 @@ namespace aexrt {
 
 namespace {
 
-constexpr int WT = 32;       // tiles per block
-constexpr int WN = 32;       // output channels per block
-constexpr int WKC = 32;      // channels per K chunk
+constexpr int WKC = 32;        // channels per K chunk of a wave
 constexpr int VROW = WKC + 8;  // padded LDS row (halves)
+constexpr uint32_t kOob = 0xFFFFFFF0u;
 
 // 4x4 input patch -> V = B^T d B for one channel (RT:2533-2548).
 __device__ __forceinline__ void input_transform(const float (&d)[4][4], float (&v)[16]) {
@@ -41,157 +40,266 @@ __device__ __forceinline__ void input_transform(const float (&d)[4][4], float (&
     }
 }
 
-// Bias, activation, residual, store and amax of one output tile: m[r] holds
-// the 16 transform points of (tile T, channel oc); out = A^T M A (RT:2612-2619).
-__device__ __forceinline__ void output_tile(const ConvParams& p, const float (&mr)[16], int T, int oc, int tiles_w,
-                                            int tiles_img, float& gmax) {
+// The four outputs of one tile and channel from its 16 points: A^T M A
+// (RT:2612-2619).
+__device__ __forceinline__ void output_transform(const float (&mr)[16], float (&o)[4]) {
     float r0[4], r1[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
         r0[q] = mr[0 * 4 + q] + mr[1 * 4 + q] + mr[2 * 4 + q];
         r1[q] = mr[1 * 4 + q] - mr[2 * 4 + q] - mr[3 * 4 + q];
     }
-    float o[4];
     o[0] = r0[0] + r0[1] + r0[2];
     o[1] = r0[1] - r0[2] - r0[3];
     o[2] = r1[0] + r1[1] + r1[2];
     o[3] = r1[1] - r1[2] - r1[3];
+}
+
+// Element offsets of tile T's first output position in the output and residual
+// views.
+struct TilePlace {
+    int64_t y, r;
+};
+__device__ __forceinline__ TilePlace tile_place(const ConvParams& p, int T, int tiles_w, int tiles_img) {
     const int n = T / tiles_img;
     const int rem = T - n * tiles_img;
-    const int ty = rem / tiles_w;
-    const int tx = rem - ty * tiles_w;
-    const float bs = p.bias[oc];
-    const bool do_silu = p.flags & kConvSilu;
+    const int ty = rem / tiles_w, tx = rem - ty * tiles_w;
+    const int64_t pos = (int64_t)ty * 2 * p.OW + tx * 2;
+    return {(int64_t)n * p.y_nstride + pos * p.y_cstride, (int64_t)n * p.r_nstride + pos * p.r_cstride};
+}
+
+// Bias, activation and residual of one output value, stored at element yo of
+// the output; returns |value| as stored.
+__device__ __forceinline__ float output_value(const ConvParams& p, float v, float bias, int64_t yo, int64_t ro) {
+    v += bias;
+    if (p.flags & kConvSilu) v = silu(v);
     const bool do_res = p.flags & kConvResidual;
-    const bool out_f32 = p.flags & kConvOutF32;
+    if (p.flags & kConvOutF32) {
+        if (do_res) v = v + __half2float(p.res[ro]);
+        reinterpret_cast<float*>(p.y)[yo] = v;
+        return fabsf(v);
+    }
+    __half h = __float2half(v);
+    if (do_res)  // fp16 conv output + fp16 residual, the reference's separate add
+        h = __float2half(__half2float(h) + __half2float(p.res[ro]));
+    reinterpret_cast<__half*>(p.y)[yo] = h;
+    return fabsf(__half2float(h));
+}
+
+// The same for four consecutive channels of one position, one access each.
+__device__ __forceinline__ float output_values4(const ConvParams& p, const float (&o)[4], const float (&bias)[4],
+                                                int64_t yo, int64_t ro) {
+    float v[4], g = 0.0f, res[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    const bool do_res = p.flags & kConvResidual;
+    if (do_res) {
+        const uint2 h = *reinterpret_cast<const uint2*>(p.res + ro);
+        const float2 lo = __half22float2(*reinterpret_cast<const __half2*>(&h.x));
+        const float2 hi = __half22float2(*reinterpret_cast<const __half2*>(&h.y));
+        res[0] = lo.x, res[1] = lo.y, res[2] = hi.x, res[3] = hi.y;
+    }
+    const bool do_silu = p.flags & kConvSilu;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        float v = o[q] + bs;
-        if (do_silu) v = silu(v);
-        const int oy = ty * 2 + (q >> 1), ox = tx * 2 + (q & 1);
-        const int64_t pos = (int64_t)oy * p.OW + ox;
-        const int64_t yo = (int64_t)n * p.y_nstride + pos * p.y_cstride + oc;
-        if (out_f32) {
-            if (do_res) v = v + __half2float(p.res[(int64_t)n * p.r_nstride + pos * p.r_cstride + oc]);
-            reinterpret_cast<float*>(p.y)[yo] = v;
-            gmax = fmaxf(gmax, fabsf(v));
-        } else {
-            __half h = __float2half(v);
-            if (do_res)  // fp16 conv output + fp16 residual, the reference's separate add
-                h = __float2half(__half2float(h) + __half2float(p.res[(int64_t)n * p.r_nstride + pos * p.r_cstride + oc]));
-            reinterpret_cast<__half*>(p.y)[yo] = h;
-            gmax = fmaxf(gmax, fabsf(__half2float(h)));
+    for (int i = 0; i < 4; ++i) {
+        v[i] = o[i] + bias[i];
+        if (do_silu) v[i] = silu(v[i]);
+    }
+    if (p.flags & kConvOutF32) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if (do_res) v[i] = v[i] + res[i];
+            g = fmaxf(g, fabsf(v[i]));
         }
+        *reinterpret_cast<float4*>(reinterpret_cast<float*>(p.y) + yo) = make_float4(v[0], v[1], v[2], v[3]);
+        return g;
+    }
+    __half h[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        h[i] = __float2half(v[i]);
+        if (do_res) h[i] = __float2half(__half2float(h[i]) + res[i]);
+        g = fmaxf(g, fabsf(__half2float(h[i])));
+    }
+    uint2 w;
+    __builtin_memcpy(&w, h, 8);
+    *reinterpret_cast<uint2*>(reinterpret_cast<__half*>(p.y) + yo) = w;
+    return g;
+}
+
+// Four channels of a 4x4 patch -> V of the tile, four halves at vs[r * rstep]
+// per transform point, written NQ channels at a time (2: half the registers).
+template <int NQ>
+__device__ __forceinline__ void transform4(const uint2 (&d)[4][4], _Float16* vs, int rstep) {
+    typedef _Float16 vh __attribute__((ext_vector_type(NQ)));
+#pragma unroll
+    for (int q0 = 0; q0 < 4; q0 += NQ) {
+        vh out[16];
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+            float dq[4][4], v[16];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const uint32_t w = q0 + q < 2 ? d[i][j].x : d[i][j].y;
+                    const float2 f = __half22float2(*reinterpret_cast<const __half2*>(&w));
+                    dq[i][j] = (q0 + q) & 1 ? f.y : f.x;
+                }
+            input_transform(dq, v);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) out[r][q] = (_Float16)v[r];
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) *reinterpret_cast<vh*>(vs + r * rstep + q0) = out[r];
+        if (NQ < 4) __builtin_amdgcn_sched_barrier(0);
     }
 }
 
-// Large maps: a block owns 32 tiles x 32 output channels; each wave computes
-// the same 16x16 (tile, oc) sub-block for all 16 points, so after the K loop
-// every lane holds all 16 points of its (tile, oc) pairs and the output
-// transform runs in registers.  V is staged in LDS per 32-channel chunk by
-// all 256 threads; U ([16][OCp][Cp] fp16, repacked at load) streams from L2.
-__global__ __launch_bounds__(256) void winograd_f2x2_kernel(ConvParams p) {
-    __shared__ __attribute__((aligned(16))) _Float16 vs[16][WT][VROW];
+// A block owns 16 TS tiles x 16 OW output channels: OW of its four waves
+// across the channels, the others across the tile subtiles.  Each wave computes
+// its (channel, tile) subtiles for all 16 points, so after the K loop a lane
+// holds every point of four consecutive channels of a tile, transforms them in
+// registers and stores 8 bytes a position.  What bounds it is latency: load a
+// patch, transform, LDS, barrier, U from L2.  So a thread issues its 16 patch
+// loads at once (out-of-range offsets read zero, no branch), the next chunk's
+// while this one is multiplied, transforms four channels and writes 8 bytes to
+// LDS per point, and a block of 16 tiles takes 64 channels a chunk.
+// 64 -> 64 at 40 x 40, 8 images: 9.3 us (14.8 with 32 tiles x 32 channels,
+// branched loads and a 2-byte LDS write per value).
+template <int TS, int OW>
+__global__ __launch_bounds__(256, TS) void winograd_f2x2_kernel(ConvParams p, int vec) {
+    constexpr int T_BLK = 16 * TS;        // tiles of the block
+    constexpr int KC = 1024 / T_BLK;      // channels of a chunk: four a thread
+    constexpr int KS = KC / 32;           // MFMA k steps of a chunk
+    constexpr int MT = TS * OW / 4;       // tile subtiles of a wave
+    constexpr int ROW = KC + 8;
+    __shared__ __attribute__((aligned(16))) _Float16 vs[16][T_BLK][ROW];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = tid >> 6;
-    const int wt = wave >> 1, wn = wave & 1;
+    const int wn = wave % OW, wt = wave / OW;
     const int lr = lane & 15, lg = lane >> 4;
 
     const int tiles_w = p.OW / 2, tiles_h = p.OH / 2;
     const int tiles_img = tiles_w * tiles_h;
     const int ttot = p.N * tiles_img;
-    const int ntn = (p.OC + WN - 1) / WN;
-    const int t0 = (blockIdx.x / ntn) * WT;
-    const int n0 = (blockIdx.x % ntn) * WN;
+    const int ntn = (p.OC + 16 * OW - 1) / (16 * OW);
+    const int b = xcd_remap(blockIdx.x, gridDim.x);
+    const int t0 = (b / ntn) * T_BLK;
+    const int n0 = (b % ntn) * 16 * OW;
 
     // transform unit of this thread: tile tl, channels c4..c4+3 of the chunk
-    const int tl = tid >> 3;
-    const int c4 = (tid & 7) * 4;
+    const int tl = tid / (KC / 4);
+    const int c4 = (tid % (KC / 4)) * 4;
     const int T = t0 + tl;
-    int y0 = 0, x0 = 0;
-    int64_t xbase = 0;
-    const bool t_ok = T < ttot;
-    if (t_ok) {
+    uint32_t base = 0, inside = 0;  // byte offset of the patch's corner; its taps inside the image
+    if (T < ttot) {
         const int n = T / tiles_img;
         const int rem = T - n * tiles_img;
         const int ty = rem / tiles_w;
-        const int tx = rem - ty * tiles_w;
-        y0 = ty * 2 - 1;
-        x0 = tx * 2 - 1;
-        xbase = (int64_t)n * p.x_nstride;
+        const int y0 = ty * 2 - 1, x0 = (rem - ty * tiles_w) * 2 - 1;
+        base = (uint32_t)((int64_t)n * p.x_nstride + ((int64_t)y0 * p.W + x0) * p.x_cstride + c4) * 2u;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if ((unsigned)(y0 + i) < (unsigned)p.H && (unsigned)(x0 + j) < (unsigned)p.W)
+                    inside |= 1u << (4 * i + j);
     }
-    const __half* xh = reinterpret_cast<const __half*>(p.x);
-    const _Float16* U = reinterpret_cast<const _Float16*>(p.w);
-    const int oc_b = n0 + wn * 16 + lr;
-    const bool oc_b_ok = oc_b < p.OCp;
-
-    v4f acc[16];
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] = v4f{0, 0, 0, 0};
-
-    const int Cp = p.Kp;
-    for (int cb = 0; cb < Cp; cb += WKC) {
-        // B operands for all 16 points (independent of LDS, issue first).
-        v8h b[16];
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            if (oc_b_ok)
-                b[r] = *reinterpret_cast<const v8h*>(U + ((int64_t)r * p.OCp + oc_b) * Cp + cb + lg * 8);
-            else
-                b[r] = v8h{0, 0, 0, 0, 0, 0, 0, 0};
-        }
-        // Input transform of 4 channels of one tile.
-        float d[4][4][4];
-        const int c = cb + c4;
+    const __amdgpu_buffer_rsrc_t rx =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p.x), 0, p.x_bytes, 0x00020000);
+    uint2 d[4][4];
+    auto load_patch = [&](int cb) {
+        const bool cok = cb + c4 < p.C;
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const int iy = y0 + i, ix = x0 + j;
-                float2 lo = make_float2(0.f, 0.f), hi = make_float2(0.f, 0.f);
-                if (t_ok && c < p.C && (unsigned)iy < (unsigned)p.H && (unsigned)ix < (unsigned)p.W) {
-                    const __half2* src = reinterpret_cast<const __half2*>(
-                        xh + xbase + ((int64_t)iy * p.W + ix) * p.x_cstride + c);
-                    lo = __half22float2(src[0]);
-                    hi = __half22float2(src[1]);
-                }
-                d[i][j][0] = lo.x; d[i][j][1] = lo.y; d[i][j][2] = hi.x; d[i][j][3] = hi.y;
+                const uint32_t off = base + (uint32_t)(i * p.W + j) * (uint32_t)p.x_cstride * 2u + (uint32_t)cb * 2u;
+                const auto v = __builtin_amdgcn_raw_buffer_load_b64(
+                    rx, cok && (inside >> (4 * i + j) & 1u) ? off : kOob, 0, 0);
+                d[i][j] = make_uint2(v[0], v[1]);
             }
-        __syncthreads();  // previous chunk's MFMAs are done with vs
+    };
+    const int Cp = p.Kp;
+    const int oc_u = min(n0 + wn * 16 + lr, p.OCp - 1);  // (rows past the last are not stored)
+    const _Float16* U = reinterpret_cast<const _Float16*>(p.w) + (int64_t)oc_u * Cp + lg * 8;
+    // the points of a k step, all at once or (with 32 accumulators a lane) half
+    constexpr int UR = MT == 1 ? 16 : 8;
+    auto load_u = [&](int c, int r0, v8h (&u)[UR]) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            float dq[4][4], v[16];
+        for (int r = 0; r < UR; ++r) u[r] = *reinterpret_cast<const v8h*>(U + (int64_t)(r0 + r) * p.OCp * Cp + c);
+    };
+
+    v4f acc[MT][16];
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+    for (int m = 0; m < MT; ++m)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) dq[i][j] = d[i][j][q];
-            input_transform(dq, v);
-#pragma unroll
-            for (int r = 0; r < 16; ++r) vs[r][tl][c4 + q] = (_Float16)v[r];
-        }
+        for (int r = 0; r < 16; ++r) acc[m][r] = v4f{0, 0, 0, 0};
+
+    // with 32 accumulators a lane has no registers for a second patch; the other
+    // block of its CU fills the wait instead
+    constexpr bool kAhead = MT == 1;
+    if (kAhead) load_patch(0);
+    for (int cb = 0; cb < Cp; cb += KC) {
+        if (!kAhead) load_patch(cb);
+        if (cb) __syncthreads();  // the previous chunk's MFMAs are done with vs
+        transform4<MT == 1 ? 4 : 2>(d, &vs[0][tl][c4], T_BLK * ROW);
+        if (kAhead && cb + KC < Cp) load_patch(cb + KC);
+        constexpr int NU = KS * 16 / UR;
+        v8h u[NU][UR];
+        load_u(cb, 0, u[0]);
         __syncthreads();
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const v8h a = *reinterpret_cast<const v8h*>(&vs[r][wt * 16 + lr][lg * 8]);
-            acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b[r], acc[r], 0, 0, 0);
+        for (int s = 0; s < NU; ++s) {
+            const int ks = s * UR / 16, r0 = s * UR % 16;
+            if (cb + ks * 32 >= Cp) break;
+            if (s + 1 < NU && cb + (s + 1) * UR / 16 * 32 < Cp)
+                load_u(cb + (s + 1) * UR / 16 * 32, (s + 1) * UR % 16, u[s + 1]);
+#pragma unroll
+            for (int r = 0; r < UR; ++r)
+#pragma unroll
+                for (int m = 0; m < MT; ++m) {
+                    const v8h v =
+                        *reinterpret_cast<const v8h*>(&vs[r0 + r][(wt * MT + m) * 16 + lr][ks * 32 + lg * 8]);
+                    acc[m][r0 + r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(u[s][r], v, acc[m][r0 + r], 0, 0, 0);
+                }
+            if (MT > 1) __builtin_amdgcn_sched_barrier(0);
         }
     }
 
-    // Lane has tiles t0 + wt*16 + lg*4 + i (i = 0..3) of output channel
-    // n0 + wn*16 + lr; point r = 4*row + col.
-    const int oc = n0 + wn * 16 + lr;
+    // lane: channels oc0 .. oc0 + 3 of tile t0 + (wt MT + m) 16 + lr; point r = 4*row + col
+    const int oc0 = n0 + wn * 16 + lg * 4;
+    float bias[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) bias[i] = oc0 + i < p.OC ? p.bias[oc0 + i] : 0.0f;
     float gmax = 0.0f;
-    if (oc < p.OC) {
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        const int Ti = t0 + (wt * MT + m) * 16 + lr;
+        if (Ti >= ttot || oc0 >= p.OC) continue;
+        float o[4][4];  // [position][channel]
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const int Ti = t0 + wt * 16 + lg * 4 + i;
-            if (Ti >= ttot) continue;
-            float mr[16];
+            float mr[16], oq[4];
 #pragma unroll
-            for (int r = 0; r < 16; ++r) mr[r] = acc[r][i];
-            output_tile(p, mr, Ti, oc, tiles_w, tiles_img, gmax);
+            for (int r = 0; r < 16; ++r) mr[r] = acc[m][r][i];
+            output_transform(mr, oq);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) o[q][i] = oq[q];
+        }
+        const TilePlace at = tile_place(p, Ti, tiles_w, tiles_img);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int64_t pos = (int64_t)(q >> 1) * p.OW + (q & 1);
+            const int64_t yo = at.y + pos * p.y_cstride + oc0, ro = at.r + pos * p.r_cstride + oc0;
+            if (vec && oc0 + 3 < p.OC) {
+                gmax = fmaxf(gmax, output_values4(p, o[q], bias, yo, ro));
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (oc0 + i < p.OC) gmax = fmaxf(gmax, output_value(p, o[q][i], bias[i], yo + i, ro + i));
+            }
         }
     }
     if (p.y_slots.p) {
@@ -263,32 +371,18 @@ __global__ __launch_bounds__(256) void winograd_f2x2_ksplit_kernel(ConvParams p)
 #pragma unroll
         for (int half = 0; half < 2; ++half) {
             const int c = cb + half * 16 + c4;
-            float d[4][4][4];
+            uint2 d[4][4];
 #pragma unroll
             for (int i = 0; i < 4; ++i)
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     const int iy = y0 + i, ix = x0 + j;
-                    float2 lo = make_float2(0.f, 0.f), hi = make_float2(0.f, 0.f);
-                    if (t_ok && c < p.C && (unsigned)iy < (unsigned)p.H && (unsigned)ix < (unsigned)p.W) {
-                        const __half2* src = reinterpret_cast<const __half2*>(
-                            xh + xbase + ((int64_t)iy * p.W + ix) * p.x_cstride + c);
-                        lo = __half22float2(src[0]);
-                        hi = __half22float2(src[1]);
-                    }
-                    d[i][j][0] = lo.x; d[i][j][1] = lo.y; d[i][j][2] = hi.x; d[i][j][3] = hi.y;
+                    d[i][j] = make_uint2(0u, 0u);
+                    if (t_ok && c < p.C && (unsigned)iy < (unsigned)p.H && (unsigned)ix < (unsigned)p.W)
+                        d[i][j] = *reinterpret_cast<const uint2*>(xh + xbase + ((int64_t)iy * p.W + ix) * p.x_cstride +
+                                                                  c);
                 }
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                float dq[4][4], v[16];
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) dq[i][j] = d[i][j][q];
-                input_transform(dq, v);
-#pragma unroll
-                for (int r = 0; r < 16; ++r) vs[r][tl][half * 16 + c4 + q] = (_Float16)v[r];
-            }
+            transform4<4>(d, &vs[0][tl][half * 16 + c4], ST * VROW);
         }
         // the region is private to this wave: LDS operations of one wave
         // complete in order, only the compiler must not move them
@@ -323,7 +417,15 @@ __global__ __launch_bounds__(256) void winograd_f2x2_ksplit_kernel(ConvParams p)
             for (int w = 0; w < 4; ++w) t += red[((w * 16 + r) * 4 + wave) * 64 + lane];
             mr[r] = t;
         }
-        output_tile(p, mr, Ti, oc, tiles_w, tiles_img, gmax);
+        float o[4];
+        output_transform(mr, o);
+        const TilePlace at = tile_place(p, Ti, tiles_w, tiles_img);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int64_t pos = (int64_t)(q >> 1) * p.OW + (q & 1);
+            gmax = fmaxf(gmax, output_value(p, o[q], p.bias[oc], at.y + pos * p.y_cstride + oc,
+                                            at.r + pos * p.r_cstride + oc));
+        }
     }
     if (p.y_slots.p) {
         gmax = wave_max(gmax);
@@ -333,18 +435,54 @@ __global__ __launch_bounds__(256) void winograd_f2x2_ksplit_kernel(ConvParams p)
 
 }  // namespace
 
-// The 32x32 block tile when it yields at least one block per CU, else the
-// k-split 16x16 tile (maps of 10x10 / 20x20 at small batch).
-hipError_t launch_winograd_f2x2(const ConvParams& p, hipStream_t stream) {
-    const int64_t ttot = (int64_t)p.N * (p.OH / 2) * (p.OW / 2);
-    const int64_t big = ((ttot + WT - 1) / WT) * ((p.OC + WN - 1) / WN);
-    if (big >= 256 || p.Kp < 4 * WKC) {
-        hipLaunchKernelGGL(winograd_f2x2_kernel, dim3((unsigned)big), dim3(256), 0, stream, p);
-    } else {
-        const int64_t small = ((ttot + 15) / 16) * ((p.OC + 15) / 16);
-        hipLaunchKernelGGL(winograd_f2x2_ksplit_kernel, dim3((unsigned)small), dim3(256), 0, stream, p);
+namespace {
+template <int TS, int OW>
+void launch_tile(const ConvParams& p, int64_t ttot, int vec, hipStream_t stream) {
+    const int64_t blocks = ((ttot + 16 * TS - 1) / (16 * TS)) * ((p.OC + 16 * OW - 1) / (16 * OW));
+    hipLaunchKernelGGL((winograd_f2x2_kernel<TS, OW>), dim3((unsigned)blocks), dim3(256), 0, stream, p, vec);
+}
+}  // namespace
+
+// Tile by the blocks it leaves.  16 tiles x 64 channels need a CU to themselves
+// (registers), so they are for launches of at most one block a CU (64 -> 64 at
+// 40 x 40 x 8: 9.3 us against 10.2 with 32 x 32; 256 -> 256 at 40 x 40 x 2: 24.8
+// against 28.8).  Beyond that 32 tiles x 64 channels, two blocks to a CU (128 ->
+// 128 at 20 x 20 x 32: 17.4 us against 27.0; 64 -> 64 at 40 x 40 x 64: 30.7, 104
+// before these tiles), and with up to 32 output channels 32 x 32.  Few tiles and
+// many channels (10x10 / 20x20 maps at small batch): the waves split the channels.
+// Inputs over 2 GB go in several launches, one image over 2 GB by 64-bit addresses.
+hipError_t launch_winograd_f2x2(const ConvParams& p0, hipStream_t stream) {
+    const int HW = p0.H * p0.W, tiles_img = (p0.OH / 2) * (p0.OW / 2);
+    const uint64_t image = std::max<uint64_t>((uint64_t)p0.x_nstride, (uint64_t)HW * p0.x_cstride) * 2;
+    const bool f32 = (p0.flags & kConvOutF32) != 0;
+    auto aligned = [](const void* q, int64_t ns, int64_t cs, uintptr_t bytes) {
+        return reinterpret_cast<uintptr_t>(q) % bytes == 0 && ns % 4 == 0 && cs % 4 == 0;
+    };
+    const int vec = aligned(p0.y, p0.y_nstride, p0.y_cstride, f32 ? 16 : 8) &&
+                    (!p0.res || aligned(p0.res, p0.r_nstride, p0.r_cstride, 8));
+    const int64_t all = (int64_t)p0.N * tiles_img;
+    const int oc64 = (p0.OC + 63) / 64;
+    if (image > kMaxViewBytes || ((all + 15) / 16 * oc64 < 128 && p0.Kp >= 4 * WKC)) {
+        const int64_t small = ((all + 15) / 16) * ((p0.OC + 15) / 16);
+        hipLaunchKernelGGL(winograd_f2x2_ksplit_kernel, dim3((unsigned)small), dim3(256), 0, stream, p0);
+        return hipGetLastError();
     }
-    return hipGetLastError();
+    const int per = (int)std::min<uint64_t>((uint64_t)p0.N, kMaxViewBytes / std::max<uint64_t>(image, 1));
+    for (int n0 = 0; n0 < p0.N; n0 += per) {
+        ConvParams p = p0;
+        p.N = std::min(per, p0.N - n0);
+        p.x = static_cast<const __half*>(p0.x) + (int64_t)n0 * p0.x_nstride;
+        p.y = static_cast<char*>(p0.y) + (int64_t)n0 * p0.y_nstride * (f32 ? 4 : 2);
+        if (p0.res) p.res = p0.res + (int64_t)n0 * p0.r_nstride;
+        p.x_bytes = (uint32_t)(((int64_t)(p.N - 1) * p.x_nstride + (int64_t)(HW - 1) * p.x_cstride + p.C) * 2);
+        const int64_t ttot = (int64_t)p.N * tiles_img;
+        if (p.OC <= 32) launch_tile<2, 2>(p, ttot, vec, stream);
+        else if ((ttot + 15) / 16 * oc64 <= 256) launch_tile<1, 4>(p, ttot, vec, stream);
+        else launch_tile<2, 4>(p, ttot, vec, stream);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 }  // namespace aexrt
