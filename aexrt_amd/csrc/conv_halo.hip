@@ -91,20 +91,18 @@ bool halo_geometry(HaloParams& h, const HaloTile& t, bool int8) {
     return true;
 }
 
-// Estimated duration (GPU clocks) of a launch with tile t.  Per tile and
-// block: MFMA issue of one wave, LDS operand reads of the 4 waves, window
-// staging (loads + int8 quantization), a fixed part per chunk (barrier,
-// latency) and per tile (epilogue).  Blocks spread over 256 CUs; the input
-// window traffic (with its halo, once per oc tile) and the output bound from
-// below.
-double halo_cost(const HaloParams& h, const HaloTile& t, bool int8) {
+// Estimated duration (GPU clocks) of a launch on the fp32 NCHW input with tile
+// t.  Per tile and block: MFMA issue of one wave, LDS operand reads of the 4
+// waves, window staging, a fixed part per chunk (barrier, latency) and per tile
+// (epilogue).  Blocks spread over 256 CUs; the input window traffic (with its
+// halo, once per oc tile) and the output bound from below.
+double halo_nchw_cost(const HaloParams& h, const HaloTile& t) {
     const ConvParams& p = h.c;
-    const int wq = int8 ? 1 : 2;
     const double steps = (double)h.nch * h.spc;
-    const double t_mfma = steps * t.jn * t.pw * wq * 16.0;
-    const double t_lds = steps * (t.jn + t.pw) * wq * 4 * 8.0;
-    const double t_stage = h.nch * std::ceil(h.npieces / 256.0) * (int8 ? 110.0 : 24.0);
-    const double t_tile = std::max(t_mfma, t_lds) + t_stage + h.nch * 350.0 + t.jn * t.pw * (int8 ? 160.0 : 120.0);
+    const double t_mfma = steps * t.jn * t.pw * 2 * 16.0;
+    const double t_lds = steps * (t.jn + t.pw) * 2 * 4 * 8.0;
+    const double t_stage = h.nch * std::ceil(h.npieces / 256.0) * 24.0;
+    const double t_tile = std::max(t_mfma, t_lds) + t_stage + h.nch * 350.0 + t.jn * t.pw * 120.0;
     const double blocks = (double)h.ntile * h.c.ntn;
     const double waves_of_blocks = std::ceil(blocks / 512.0);  // ~2 blocks per CU overlap
     const double compute = waves_of_blocks * t_tile;
@@ -121,38 +119,31 @@ bool halo_shape_ok(const ConvParams& p, bool int8) {
     return p.loader == kLoaderNhwc && p.C % (int8 ? 16 : 8) == 0 && p.x_cstride % 8 == 0;
 }
 
-// Lowest-cost tile of the instantiated shapes.
-bool choose_halo_tile(HaloParams& h, bool int8, HaloTile& best) {
+// Lowest-cost tile for the fp32 NCHW input (one chunk: its 8 padded channels).
+bool choose_nchw_tile(HaloParams& h, HaloTile& best) {
     const ConvParams& p = h.c;
     double best_cost = 0.0;
     bool found = false;
     const int ocj = (p.OCp + 15) / 16;
-    const bool nchw = p.loader == kLoaderNchwF32;
-    for (int div = 1; div <= 8; div <<= 1) {
-        if (p.C % div) break;
-        const int CC = p.C / div;
-        if (CC % (int8 ? 16 : 8) || CC > (int8 ? 128 : 64)) continue;
-        for (int jn = 1; jn <= std::min(4, pow2_at_least(ocj, 4)); jn <<= 1) {
-            for (int pw = nchw ? 2 : 1; pw <= 4; pw <<= 1) {
-                // the whole row, or its width rounded up to 4 (the NCHW
-                // loader needs TC * S % 4 == 0), or multiples of 16
-                const int ow4 = (p.OW + 3) / 4 * 4;
-                int tcs[7] = {p.OW, ow4, 16, 32, 48, 64, 80};
-                for (int tc : tcs) {
-                    if (tc > ow4 || (tc > p.OW && tc != ow4) || (tc < p.OW && tc > 64 * pw)) continue;
-                    const int TR = std::min(p.OH, 64 * pw / tc);
-                    if (TR < 1) continue;
-                    for (int np : {4, 8}) {
-                        const HaloTile t{jn, pw, np, TR, tc, CC};
-                        HaloParams hh = h;
-                        if (!halo_geometry(hh, t, int8)) continue;
-                        if (np == 8 && hh.npieces <= 4 * 64 * t.nw) continue;
-                        const double c = halo_cost(hh, t, int8);
-                        if (!found || c < best_cost) {
-                            best_cost = c;
-                            best = t;
-                            found = true;
-                        }
+    for (int jn = 1; jn <= std::min(4, pow2_at_least(ocj, 4)); jn <<= 1) {
+        for (int pw = 2; pw <= 4; pw <<= 1) {
+            // the whole row, its width rounded up to 4 (the loader needs TC * S % 4 == 0), or multiples of 16
+            const int ow4 = (p.OW + 3) / 4 * 4;
+            int tcs[7] = {p.OW, ow4, 16, 32, 48, 64, 80};
+            for (int tc : tcs) {
+                if (tc > ow4 || (tc > p.OW && tc != ow4) || (tc < p.OW && tc > 64 * pw)) continue;
+                const int TR = std::min(p.OH, 64 * pw / tc);
+                if (TR < 1) continue;
+                for (int np : {4, 8}) {
+                    const HaloTile t{jn, pw, np, TR, tc, p.C};
+                    HaloParams hh = h;
+                    if (!halo_geometry(hh, t, false)) continue;
+                    if (np == 8 && hh.npieces <= 4 * 64 * t.nw) continue;
+                    const double c = halo_nchw_cost(hh, t);
+                    if (!found || c < best_cost) {
+                        best_cost = c;
+                        best = t;
+                        found = true;
                     }
                 }
             }
@@ -262,6 +253,11 @@ bool set_conv3x3_halo(int mode, int jn, int pw, int tr, int tc, int cc) {
     return true;
 }
 
+bool halo_mode_auto() {
+    const int mode = g_halo_mode.load(std::memory_order_relaxed);
+    return mode != 1 && mode != 2;
+}
+
 bool forced_wide_choice(ConvChoice& c) {
     if (g_halo_mode.load(std::memory_order_relaxed) != 4) return false;
     const uint64_t f = g_force.load(std::memory_order_relaxed);
@@ -311,8 +307,8 @@ hipError_t launch_conv_halo(const ConvParams& p, bool int8, int epi, hipStream_t
             HaloParams h8 = h;
             if (!halo_geometry(h8, t, int8)) return hipErrorInvalidValue;
         }
-    } else if (!choose_halo_tile(h, int8, t)) {
-        return hipErrorNotSupported;
+    } else if (p.loader != kLoaderNchwF32 || !choose_nchw_tile(h, t)) {
+        return hipErrorNotSupported;  // NHWC tiles are chosen by the caller
     }
     if (!halo_geometry(h, t, int8)) return hipErrorNotSupported;
     return halo_launch(h, int8, epi, t, stream);

@@ -2,8 +2,11 @@
 // choice, batch splitting for 32-bit view offsets, launch parameters.
 #include <algorithm>
 #include <atomic>
-
+#include <cmath>
 #include <cstdio>
+#include <cstring>
+#include <vector>
+
 #include "conv_igemm.h"
 
 namespace aexrt {
@@ -154,15 +157,203 @@ int enumerate_conv_choices(const ConvParams& p, bool int8, ConvChoice* out, int 
     return n;
 }
 
+namespace {
+
+// ---- 3x3 convs without a measured tile ----------------------------------------
+// Every tile that the three 3x3 kernels (halo window, 32x32 MFMA, implicit
+// GEMM) offer for the conv is given an estimated time, and the fastest runs.
+// The estimate weighs what a launch does on its most loaded CU (weight bytes
+// staged, matrix-core and LDS-read clocks, conversion work, input bytes of all
+// blocks) and the serial chain of one block (iterations, their MFMA clocks and
+// staging rounds, position tiles).  In the halo and the plain implicit-GEMM
+// kernel several blocks share a CU and cover each other's chains, so the longer
+// of the two counts; the other two run them one after the other.
+//
+// The rates below are microseconds per unit, fitted (non-negative least
+// squares) to 38800 measured launches: 642 random shapes (batch 1-64, maps
+// 4-160, 8-512 channels, strides 1 and 2) with all of their tiles.  Over those
+// shapes the chosen tile takes 1.02x (int8) and 1.03x (fp16) the time of the
+// best one (the same on shapes left out of the fit).  The rule before it (halo
+// tiles of 4 waves by a clock count, implicit GEMM only where no halo tile fits)
+// took 1.15x: 4 waves leave a CU half empty where the weights fill the LDS, and
+// it never took the 32x32-MFMA kernel.  Examples, us before and after: int8
+// 64 -> 128 channels at 80x80 from 160x160 x32 81.8 -> 69.7, 256 at 40x40 x2 17.9
+// -> 11.4, 512 at 20x20 38.7 -> 14.4; fp16 128 at 80x80 x4 29.5 -> 22.6, 256 -> 64
+// at 20x20 x8 17.1 -> 10.8.
+struct TileRates {
+    double base;      // launch and first loads
+    double weights;   // per 10 KB of weights staged on the CU
+    double mfma;      // per 10k matrix-core clocks of the CU's blocks
+    double lds;       // per 10k LDS-read clocks of the CU's blocks
+    double convert;   // per 1k wave-rounds of conversion (16 bytes a lane) on a SIMD
+    double bytes;     // per 100 MB of input read by all blocks
+    double epilogue;  // per 100 position x channel subtiles stored by the CU
+    double iter;      // per 10 iterations (barrier, latency) of a block
+    double chain;     // per 10k matrix-core clocks in one block's chain
+    double rounds;    // per 100 staging rounds in one block's chain
+    double tile;      // per 10 position tiles of a block
+    bool overlap;     // the CU's work and a block's chain cover each other
+};
+// halo, 32x32 MFMA, implicit GEMM, implicit GEMM with k split over the waves
+constexpr TileRates kRatesI8[4] = {{3.85, 0.21, 0, 3.46, 96.18, 0.33, 12.66, 0.95, 5.92, 14.76, 0.72, true},
+                                   {3.66, 0.18, 7.01, 0, 40.61, 5.25, 24.7, 0, 0.04, 14.18, 6.94, false},
+                                   {4.94, 0.21, 0, 0, 22.61, 0.48, 11.36, 3.5, 12.36, 7.39, 0, true},
+                                   {3.81, 0, 0, 0, 16.53, 2.53, 22.57, 2.16, 44.24, 0, 14.31, false}};
+constexpr TileRates kRatesF16[4] = {{3.4, 0.19, 0, 4.42, 56.91, 0.04, 12.07, 0.32, 7.99, 12.56, 0, true},
+                                    {3.47, 0.19, 8.64, 0, 0, 6.21, 36.97, 0, 0, 10.27, 0, false},
+                                    {4.18, 0.17, 0.13, 0.69, 13.35, 1.73, 7.84, 2.34, 9.51, 6.35, 0, true},
+                                    {3.25, 0, 0, 0, 15.52, 2.63, 23.49, 1.05, 41.36, 0, 14.9, false}};
+
+int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+// Estimated microseconds of a 3x3 conv with tile c (as an enumerate_* function gives it).
+double tile_time(const ConvParams& p, bool int8, const ConvChoice& c) {
+    constexpr int kCus = 256, kLds = 160 * 1024;
+    const int esz = int8 ? 1 : 2, wq = int8 ? 1 : 2;
+    // registers of the instance, as the compiler gives them within a few
+    auto waves_per_simd = [](double regs) { return 512 / (((int)(std::min(regs, 504.0) + 0.5) + 7) / 8 * 8); };
+    double wbytes, mfma, lds, convert, bytes, epilogue, iters, chain, rounds, tiles;
+    int family;
+    if (c.kind == 1) {
+        family = c.ksw ? 3 : 2;
+        const int nks = p.Kp / 64, kc = igemm::chunk_steps_of(int8, c.jn, c.ksw != 0);
+        const bool mc = nks > kc;
+        const int chunk = kc * c.jn * 16 * 64 * esz;
+        const double regs = (int8 ? 48 : 40) + (mc ? 20 : 0) + (c.ksw ? 20 : 17) * c.pw + 3.5 * c.jn * (c.pw + 1);
+        const int res = std::max(1, std::min(kLds / (chunk * (mc ? 2 : 1) + 8400), waves_per_simd(regs)));
+        const int64_t npt = cdiv(p.M, (c.ksw ? 16 : 64) * c.pw), ntn = cdiv(p.OCp / 16, c.jn);
+        int64_t groups = npt;
+        if (!c.ksw && npt * ntn > (int64_t)res * kCus) groups = std::max<int64_t>(1, (int64_t)res * kCus / ntn);
+        const double per = (double)cdiv(npt, groups);
+        const double blocks = (double)cdiv(npt, (int64_t)per) * ntn;
+        // a k-split grid may need several rounds of resident blocks
+        const double load = c.ksw && blocks > (double)kCus * res ? blocks / kCus : std::ceil(blocks / kCus);
+        const double turns = per * (c.ksw ? std::ceil(blocks / ((double)kCus * res)) : 1.0);
+        const double step = c.jn * c.pw * wq * 16.0, split = c.ksw ? 1.0 : 4.0;
+        wbytes = load * c.jn * 16.0 * nks * 64 * esz * (mc ? per : 1.0);
+        mfma = load * per * nks * step / (c.ksw ? 4.0 : 1.0);
+        lds = load * per * nks * c.jn * wq * 8.0 * split;
+        convert = load * per * nks * c.pw * 2.0 * split;
+        bytes = blocks * per * (c.ksw ? 16 : 64) * c.pw * nks * 128.0;
+        epilogue = load * per * c.jn * c.pw;
+        iters = turns * (c.ksw ? cdiv(nks, 4) : nks);
+        chain = iters * step;
+        rounds = iters * c.pw;
+        tiles = turns;
+    } else {
+        const bool m = c.kind == 5;
+        family = m ? 1 : 0;
+        const int ir = (c.tr - 1) * p.S + 3, icol = (c.tc - 1) * p.S + 3, nch = p.C / c.cc;
+        const int np = ir * icol * c.cc / (m && int8 ? 16 : 8) <= 4 * 64 * c.nw ? 4 : 8;
+        const int64_t ntile = (int64_t)p.N * cdiv(p.OH, c.tr) * cdiv(p.OW, c.tc);
+        const int jp = c.jn * c.pw;
+        double wb, tb, regs, step;
+        int64_t ntn;
+        if (m) {
+            const int64_t steps = cdiv(9 * c.cc, int8 ? 32 : 16);
+            wb = (double)nch * steps * 2 * c.jn * 32 * 16;
+            tb = (double)ir * icol * c.cc * esz;
+            ntn = cdiv(p.OCp, 32 * c.jn);
+            step = (double)steps * jp * 32;
+            lds = (double)steps * (c.jn + c.pw) * 8;
+            regs = int8 ? 23 + 18 * jp + 16.3 * c.jn + 13.6 * c.pw + 11.2 * np
+                        : 13 + 15.5 * jp + 19 * c.jn + 16.5 * c.pw + 7 * np;
+            epilogue = c.nw / 4.0;
+        } else {
+            const int64_t steps = cdiv(9 * c.cc, 64);
+            wb = (double)nch * steps * wq * c.jn * 1024;
+            const int px = c.cc * esz;
+            tb = (double)ir * icol * (px + (px / 16 % 2 ? 0 : 16));
+            ntn = cdiv(p.OCp / 16, c.jn);
+            step = (double)steps * jp * wq * 16;
+            lds = (double)steps * (c.jn + c.pw) * wq * 8;
+            regs = int8 ? 23 + 6 * jp + 11 * c.jn + 11.5 * c.pw + 8 * np
+                        : 40 + 19 * jp + 6.5 * c.jn + 11.6 * c.pw + 7 * np;
+            epilogue = jp * c.nw / 4.0;
+        }
+        const int res = std::max(1, std::min(kLds / (int)(wb + 2 * tb + 2048), waves_per_simd(regs) * 4 / c.nw));
+        int64_t groups = ntile;
+        if (ntile * ntn > (int64_t)res * kCus) groups = std::max<int64_t>(1, (int64_t)res * kCus / ntn);
+        tiles = (double)cdiv(ntile, groups);
+        const double blocks = (double)cdiv(ntile, (int64_t)tiles) * ntn;
+        const double load = std::ceil(blocks / kCus);
+        iters = tiles * nch;
+        chain = iters * step * c.nw / 4.0;
+        wbytes = load * wb;
+        mfma = load * chain;
+        lds *= load * iters * c.nw;
+        convert = load * iters * ((double)ir * icol * c.cc / 8) / 256;
+        bytes = blocks * iters * ((double)ir * icol * c.cc) * 2.0;
+        epilogue *= load * tiles;
+        rounds = iters * np;
+    }
+    const TileRates& r = (int8 ? kRatesI8 : kRatesF16)[family];
+    const double cu = r.mfma * mfma * 1e-4 + r.lds * lds * 1e-4 + r.convert * convert * 1e-3 + r.bytes * bytes * 1e-8;
+    const double block = r.iter * iters * 0.1 + r.chain * chain * 1e-4 + r.rounds * rounds * 1e-2 + r.tile * tiles * 0.1;
+    return r.base + r.weights * wbytes * 1e-4 + r.epilogue * epilogue * 1e-2 +
+           (r.overlap ? std::max(cu, block) : cu + block);
+}
+
+// Fastest estimated tile of a 3x3 conv; false (best as it was) where none applies.  With
+// a tile forced on the implicit GEMM that kernel is not among them (it runs,
+// with the forced tile, where no window kernel fits).
+bool choose_conv3x3(const ConvParams& p, bool int8, ConvChoice& best) {
+    if (p.KH != 3 || p.KW != 3 || p.P != 1 || p.loader != kLoaderNhwc || p.fuse_1x1 || p.yup || p.xup) return false;
+    // the choice is a function of the sizes below alone: the last ones of this
+    // thread are kept (enumerating the tiles takes as long as a small conv)
+    struct Entry {
+        int key[10];
+        ConvChoice best;
+        bool found;
+    };
+    constexpr int kEntries = 64;
+    static thread_local Entry memo[kEntries] = {};  // a zeroed key has N = 0: no conv's
+    const int key[10] = {p.N, p.C, p.H, p.W, p.OC, p.OH, p.OW, p.S, p.Kp, (int)int8 | (tile_forced() ? 2 : 0) |
+                         (p.x_cstride % 8 ? 4 : 0)};
+    uint32_t h = 2166136261u;
+    for (int v : key) h = (h ^ (uint32_t)v) * 16777619u;
+    Entry& e = memo[(h ^ (h >> 16)) % kEntries];
+    if (std::memcmp(e.key, key, sizeof(key)) != 0) {
+        thread_local std::vector<ConvChoice> all(kMaxConvChoices);
+        const int n = enumerate_conv_choices(p, int8, all.data(), kMaxConvChoices);
+        const ConvTile usual_tile = choose_conv_tile(p.M, p.OC, p.Kp);
+        double best_t = 0.0;
+        e.found = false;
+        for (int i = 0; i < n; ++i) {
+            const ConvChoice& c = all[i];
+            if (c.kind != 1 && c.kind != 2 && c.kind != 5) continue;
+            if (c.kind == 1) {
+                // fp16: the estimate orders the plain implicit-GEMM tiles of large maps
+                // wrongly (up to 1.4x), choose_conv_tile does not
+                const bool usual = c.jn == usual_tile.jn && c.pw == usual_tile.pw && (c.ksw != 0) == usual_tile.ksw;
+                if (tile_forced() || (int8 ? c.pw > 2 : !c.ksw && !usual)) continue;
+            } else if (c.pw > 2 || (c.kind == 2 && c.jn > 4)) {
+                continue;  // halo tiles of 5 channel subtiles with 2 position subtiles use scratch memory
+            }
+            // 32x32 MFMA: the widest tiles and the two-group blocks were the fastest at
+            // a handful of shapes only, 8 waves of 4 subtiles lose up to 1.4x to others
+            if (c.kind == 5 && (c.jn > 3 || c.ksw || (c.nw == 8 && c.jn * c.pw >= 4))) continue;
+            const double t = tile_time(p, int8, c);
+            if (!e.found || t < best_t) {
+                best_t = t;
+                e.best = c;
+                e.found = true;
+            }
+        }
+        std::memcpy(e.key, key, sizeof(key));
+    }
+    if (e.found) best = e.best;
+    return e.found;
+}
+
+}  // namespace
+
 hipError_t launch_conv_igemm(const ConvParams& p0, bool int8, hipStream_t stream) {
     const bool nchw = p0.loader == kLoaderNchwF32;
     if ((p0.loader != kLoaderNhwc && !nchw) || p0.OC % 4 || p0.C % 8 || p0.Kp % 64 || p0.OCp % 16)
         return hipErrorInvalidValue;
     if (nchw && (int8 || p0.c_real < 1 || p0.c_real > 4 || p0.x_nstride != (int64_t)p0.c_real * p0.H * p0.W))
         return hipErrorInvalidValue;
-    const ConvTile t = p0.choice.kind == 1 ? ConvTile{p0.choice.jn, p0.choice.pw, p0.choice.ksw != 0}
-                                           : choose_conv_tile(p0.M, p0.OC, p0.Kp);
-    if (p0.choice.kind == 1 && !tile_instantiated(t)) return hipErrorInvalidValue;
     const bool out_f32 = (p0.flags & kConvOutF32) != 0;
     const int HWi = p0.H * p0.W, HWo = p0.OH * p0.OW;
     // Images per launch: every view a launch touches must stay inside
@@ -185,6 +376,19 @@ hipError_t launch_conv_igemm(const ConvParams& p0, bool int8, hipStream_t stream
     if (int8 && (p0.x_slots.p == nullptr ||
                  (int64_t)p0.x_slots.stripes * p0.x_nslots > igemm::kMaxSlotReads))
         return hipErrorInvalidValue;
+    // no measured tile and none forced: a 3x3 conv's by its estimated times
+    ConvChoice choice = p0.choice;
+    ConvChoice forced_tile;
+    if (choice.kind == 0 && halo_mode_auto() && !forced_m32_choice(forced_tile) &&
+        (int8 || !forced_wide_choice(forced_tile))) {
+        ConvParams slice = p0;
+        slice.N = std::min(per_launch, p0.N);
+        slice.M = slice.N * HWo;
+        choose_conv3x3(slice, int8, choice);
+    }
+    const ConvTile t = choice.kind == 1 ? ConvTile{choice.jn, choice.pw, choice.ksw != 0}
+                                        : choose_conv_tile(p0.M, p0.OC, p0.Kp);
+    if (choice.kind == 1 && !tile_instantiated(t)) return hipErrorInvalidValue;
     const bool mc = nks > igemm::chunk_steps_of(int8, t.jn, t.ksw);
     const int f = p0.flags & (kConvSilu | kConvResidual | kConvOutF32);
     // the int32 accumulator output (acc_out) is written by the run-time
@@ -200,6 +404,7 @@ hipError_t launch_conv_igemm(const ConvParams& p0, bool int8, hipStream_t stream
         return hipErrorInvalidValue;
     for (int nb = 0; nb < p0.N; nb += per_launch) {
         ConvParams p = p0;
+        p.choice = choice;
         ConvParams f2;  // the fused 1x1 on this slice of the batch
         if (p0.fuse_1x1) {
             f2 = *p0.fuse_1x1;

@@ -202,6 +202,8 @@ int enumerate_halo_choices(const ConvParams& p, bool int8, ConvChoice* out, int 
 // (and quantized) once in LDS.  epi: 0 any flags, 1 SiLU -> fp16, 2 int8
 // SiLU + residual -> fp16.  hipErrorNotSupported for other shapes.
 hipError_t launch_conv_halo(const ConvParams& p, bool int8, int epi, hipStream_t stream);
+// False while set_conv3x3_halo turns the halo-tile kernel off or forces its tile.
+bool halo_mode_auto();
 // Halo kernel selection for 3x3 convs: mode 0 automatic, 1 never (implicit
 // GEMM only), 2 forced tile (jn oc subtiles, pw position subtiles per wave,
 // tr x tc output positions per tile, cc channels per chunk; a 3x3 conv the
