@@ -29,6 +29,11 @@
 // only, CC = 8).  Quads start at columns that are multiples of 4 (TC * S % 4
 // == 0 keeps that the same for every tile), so a quad is either wholly left
 // of the image or starts inside it.
+//
+// PG: int8 with an activation scale per 16 input channels (pg16).  Chunks of
+// 16 channels (three 64-k steps of four taps each) make every chunk one group:
+// its window is quantized with the group's scale, and its exact int32 sums are
+// scaled into fp32 accumulators at the chunk's end.
 #pragma once
 #include "conv_igemm.h"
 
@@ -59,6 +64,8 @@ constexpr int kHaloMaxSpc = 32;
 // 16-byte weight pieces per thread: the block's weights are at most
 // 64 * NW * kHaloWeightRounds * 16 bytes (64 KB with 4 waves, 128 KB with 8).
 constexpr int kHaloWeightRounds = 16;
+// Most 16-channel groups of a pg16 conv (their weights fill 128 KB of LDS at 42).
+constexpr int kHaloPgGroups = 48;
 
 namespace halo {
 
@@ -72,7 +79,7 @@ using igemm::v2i;
 using igemm::xcd_remap;
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
-template <bool INT8, int JN, int PW, int NP, int EPI, bool NCHW = false, int NW = 4>
+template <bool INT8, int JN, int PW, int NP, int EPI, bool NCHW = false, int NW = 4, bool PG = false>
 __global__ __launch_bounds__(NW * 64) void conv3x3_halo_kernel(HaloParams h) {
     constexpr int NT = NW * 64;  // threads of the block
     const ConvParams& p = h.c;
@@ -82,6 +89,7 @@ __global__ __launch_bounds__(NW * 64) void conv3x3_halo_kernel(HaloParams h) {
     constexpr int PIECE = 8 * ESZ;       // LDS bytes of one 8-channel input piece
     static_assert(JN >= 1 && JN <= 8, "JN must be 1..8");
     static_assert(!(NCHW && INT8), "the NCHW input loader is fp16 only");
+    static_assert(!PG || (INT8 && EPI == igemm::kEpiAny), "pg16: int8, any flags");
     typedef typename std::conditional<INT8, v4i, v4f>::type acc_t;
 
     // [weights: wbytes][window buffer 0: tbytes][window buffer 1: tbytes]
@@ -91,6 +99,9 @@ __global__ __launch_bounds__(NW * 64) void conv3x3_halo_kernel(HaloParams h) {
     __shared__ int l_toff[kHaloMaxSpc * 4 * WQ];
     __shared__ float l_bias[R], l_scale[R];
     __shared__ uint32_t l_slots[JN];
+    // PG: amax bits, 127 / amax and amax / 127 of every 16-channel group
+    __shared__ uint32_t l_gmax[PG ? kHaloPgGroups : 1];
+    __shared__ float l_gq[PG ? kHaloPgGroups : 1], l_gs[PG ? kHaloPgGroups : 1];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -113,7 +124,7 @@ __global__ __launch_bounds__(NW * 64) void conv3x3_halo_kernel(HaloParams h) {
 
     // ---- prologue loads: input scale, per-channel constants ----------------
     uint32_t slot_raw[igemm::kMaxSlotReads / 64];
-    if constexpr (INT8) igemm::in_slot_loads(p, lane, slot_raw);
+    if constexpr (INT8 && !PG) igemm::in_slot_loads(p, lane, slot_raw);
     const rsrc_t rb = make_rsrc(p.bias, (uint32_t)p.OC * 4u);
     const rsrc_t rsc = make_rsrc(p.w_scale, INT8 ? (uint32_t)p.OC * 4u : 0u);
     const uint32_t cofs = tid < R && n0 + tid < p.OC ? (uint32_t)(n0 + tid) * 4u : kOob;
@@ -233,7 +244,7 @@ __global__ __launch_bounds__(NW * 64) void conv3x3_halo_kernel(HaloParams h) {
     // carry the same sequence, so the prologue issues the stores of an
     // iteration too, all out of range (dropped).
 #pragma unroll
-    for (int d = 0; d < JN * PW * (EPI == igemm::kEpiAny && INT8 ? 2 : 1); ++d)
+    for (int d = 0; d < JN * PW * (EPI == igemm::kEpiAny && INT8 && !PG ? 2 : 1); ++d)
         __builtin_amdgcn_raw_buffer_store_b64(v2i{0, 0}, ry, kOob, 0, 0);
 
     // ---- tables (ALU only while the loads are in flight) -------------------
@@ -272,10 +283,29 @@ __global__ __launch_bounds__(NW * 64) void conv3x3_halo_kernel(HaloParams h) {
     }
     if (tid < JN) l_slots[tid] = 0u;
     float s_q = 0.0f, in_scale = 0.0f;
-    if constexpr (INT8) igemm::in_slot_scale(slot_raw, s_q, in_scale);
+    if constexpr (INT8 && !PG) igemm::in_slot_scale(slot_raw, s_q, in_scale);
     if (tid < R) {
         l_bias[tid] = bias_v;
-        if constexpr (INT8) l_scale[tid] = in_scale * scale_v;
+        if constexpr (INT8) l_scale[tid] = PG ? scale_v : in_scale * scale_v;
+    }
+    if constexpr (PG) {
+        // group maxima over the copies of the slot array: a run of copies a
+        // thread, then one LDS atomic each
+        if (tid < kHaloPgGroups) l_gmax[tid] = 0u;
+        __syncthreads();
+        const int row = (int)fdiv((uint32_t)tid, p.fd_ns), g = tid - row * h.nch, rows = NT / h.nch;
+        if (row < rows) {
+            uint32_t v = 0u;
+            for (uint32_t c = row; c < p.x_slots.stripes; c += rows) v = max(v, p.x_slots.p[c * p.x_slots.stride + g]);
+            if (v) atomicMax(&l_gmax[g], v);
+        }
+        __syncthreads();
+        if (tid < h.nch) {
+            const float a = u2f(l_gmax[tid]);
+            l_gs[tid] = a / 127.0f;
+            l_gq[tid] = a > 0.0f ? 127.0f / a : 0.0f;
+        }
+        __syncthreads();
     }
     if constexpr (NCHW) {
         // the padding channels of the window pixels are never written
@@ -309,6 +339,13 @@ __global__ __launch_bounds__(NW * 64) void conv3x3_halo_kernel(HaloParams h) {
     for (int j = 0; j < JN; ++j)
 #pragma unroll
         for (int q = 0; q < PW; ++q) acc[j][q] = acc_t{0, 0, 0, 0};
+    v4f accf[PG ? JN : 1][PG ? PW : 1];  // PG: scaled sums of the groups so far
+    if constexpr (PG) {
+#pragma unroll
+        for (int j = 0; j < JN; ++j)
+#pragma unroll
+            for (int q = 0; q < PW; ++q) accf[j][q] = v4f{0, 0, 0, 0};
+    }
     // packed outputs of the last finished tile (fp16: .xy; fp32: all four)
     v4i ov[JN][PW];
 
@@ -322,6 +359,7 @@ __global__ __launch_bounds__(NW * 64) void conv3x3_halo_kernel(HaloParams h) {
     int tl = 0, ch = 0;
     for (int i = 0; i < total; ++i) {
         uint8_t* const tb = win + (i & 1) * h.tbytes;
+        if constexpr (PG) s_q = l_gq[ch];
         // this iteration's window -> LDS (int8: quantized once here)
 #pragma unroll
         for (int k = 0; k < NP; ++k) {
@@ -422,6 +460,19 @@ __global__ __launch_bounds__(NW * 64) void conv3x3_halo_kernel(HaloParams h) {
             __builtin_amdgcn_sched_barrier(0);
         }
         if (s < h.spc) mma(A0, B0);
+        if constexpr (PG) {
+            // the chunk is one group: its exact sums, scaled, on top of the others'
+            const float gs = l_gs[ch];
+#pragma unroll
+            for (int j = 0; j < JN; ++j)
+#pragma unroll
+                for (int q = 0; q < PW; ++q) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        accf[j][q][r] = __builtin_fmaf((float)acc[j][q][r], gs, accf[j][q][r]);
+                    acc[j][q] = acc_t{0, 0, 0, 0};
+                }
+        }
 
         // ---- epilogue: values (VALU, at a tile's end), then the stores,
         // issued on every iteration (out of range unless at a tile's end) ----
@@ -439,7 +490,8 @@ __global__ __launch_bounds__(NW * 64) void conv3x3_halo_kernel(HaloParams h) {
 #pragma unroll
                 for (int q = 0; q < PW; ++q) {
                     float v[4];
-                    igemm::epi_values<INT8, EPI>(p, acc[j][q], bv, wv, rv[j][q], v);
+                    if constexpr (PG) igemm::epi_values<INT8, EPI>(p, accf[j][q], bv, wv, rv[j][q], v);
+                    else igemm::epi_values<INT8, EPI>(p, acc[j][q], bv, wv, rv[j][q], v);
                     const float m4 = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
                     gmax[j] = fmaxf(gmax[j], oc_ok && yo[q] >= 0 ? m4 : 0.0f);
                     if (out_f32) {
@@ -465,7 +517,7 @@ __global__ __launch_bounds__(NW * 64) void conv3x3_halo_kernel(HaloParams h) {
                 else
                     __builtin_amdgcn_raw_buffer_store_b64(v2i{ov[j][q][0], ov[j][q][1]}, ry,
                                                           ok ? (uint32_t)(yo[q] + oc0) * 2u : kOob, 0, 0);
-                if constexpr (INT8 && EPI == igemm::kEpiAny) {
+                if constexpr (INT8 && EPI == igemm::kEpiAny && !PG) {
                     // int32 accumulators (acc_out; a zero-byte view drops them)
                     const v4i av{(int)acc[j][q][0], (int)acc[j][q][1], (int)acc[j][q][2], (int)acc[j][q][3]};
                     __builtin_amdgcn_raw_buffer_store_b128(av, racc, ok ? (uint32_t)(mo[q] * p.OC + oc0) * 4u : kOob,
@@ -477,7 +529,10 @@ __global__ __launch_bounds__(NW * 64) void conv3x3_halo_kernel(HaloParams h) {
 #pragma unroll
             for (int j = 0; j < JN; ++j)
 #pragma unroll
-                for (int q = 0; q < PW; ++q) acc[j][q] = acc_t{0, 0, 0, 0};
+                for (int q = 0; q < PW; ++q) {
+                    if constexpr (PG) accf[j][q] = v4f{0, 0, 0, 0};
+                    else acc[j][q] = acc_t{0, 0, 0, 0};
+                }
         }
         tl = ntl_;
         ch = nch_;
@@ -487,11 +542,11 @@ __global__ __launch_bounds__(NW * 64) void conv3x3_halo_kernel(HaloParams h) {
 }
 
 // Blocks of one instance the GPU holds at once with lds_bytes of dynamic LDS.
-template <bool INT8, int JN, int PW, int NP, int EPI, bool NCHW, int NW>
+template <bool INT8, int JN, int PW, int NP, int EPI, bool NCHW, int NW, bool PG = false>
 int halo_resident_blocks(int lds_bytes) {
     int per_cu = 0, cus = 0, dev = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, conv3x3_halo_kernel<INT8, JN, PW, NP, EPI, NCHW, NW>, NW * 64,
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, conv3x3_halo_kernel<INT8, JN, PW, NP, EPI, NCHW, NW, PG>, NW * 64,
                                                      (size_t)lds_bytes) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || per_cu < 1 ||
         cus < 1)
@@ -501,17 +556,17 @@ int halo_resident_blocks(int lds_bytes) {
 
 // Persistent grid: every resident block slot gets one contiguous run of
 // position tiles of one oc tile.
-template <bool INT8, int JN, int PW, int NP, int EPI, bool NCHW = false, int NW = 4>
+template <bool INT8, int JN, int PW, int NP, int EPI, bool NCHW = false, int NW = 4, bool PG = false>
 hipError_t halo_launch_cfg(HaloParams h, hipStream_t stream) {
     const int lds_bytes = h.wbytes + 2 * h.tbytes;
-    const int cap = halo_resident_blocks<INT8, JN, PW, NP, EPI, NCHW, NW>(lds_bytes);
+    const int cap = halo_resident_blocks<INT8, JN, PW, NP, EPI, NCHW, NW, PG>(lds_bytes);
     int groups = h.ntile;
     if ((int64_t)h.ntile * h.c.ntn > cap) groups = std::max(1, cap / h.c.ntn);
     h.c.per = (h.ntile + groups - 1) / groups;
     groups = (h.ntile + h.c.per - 1) / h.c.per;
     const int64_t blocks = (int64_t)groups * h.c.ntn;
     if (blocks > INT32_MAX) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((conv3x3_halo_kernel<INT8, JN, PW, NP, EPI, NCHW, NW>), dim3((unsigned)blocks), dim3(NW * 64),
+    hipLaunchKernelGGL((conv3x3_halo_kernel<INT8, JN, PW, NP, EPI, NCHW, NW, PG>), dim3((unsigned)blocks), dim3(NW * 64),
                        (size_t)lds_bytes, stream, h);
     return hipGetLastError();
 }
@@ -542,6 +597,9 @@ hipError_t halo_launch_family(const HaloParams& h, int jn, int pw, int np, int n
 #undef AEXRT_HALO_CASE8
     return hipErrorInvalidValue;
 }
+
+// pg16 conv (a scale per 16 input channels): chunks of one group.
+hipError_t halo_launch_pg(const HaloParams& h, int jn, int pw, int np, int nw, hipStream_t stream);
 
 // The first conv on the fp32 NCHW input (fp16, SiLU).
 hipError_t halo_launch_nchw(const HaloParams& h, int jn, int pw, int np, hipStream_t stream);

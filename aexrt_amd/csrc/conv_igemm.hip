@@ -207,7 +207,9 @@ constexpr TileRates kRatesF16[4] = {{3.4, 0.19, 0, 4.42, 56.91, 0.04, 12.07, 0.3
 int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // Estimated microseconds of a 3x3 conv with tile c (as an enumerate_* function gives it).
-double tile_time(const ConvParams& p, bool int8, const ConvChoice& c) {
+}  // namespace
+
+double conv_tile_time(const ConvParams& p, bool int8, const ConvChoice& c) {
     constexpr int kCus = 256, kLds = 160 * 1024;
     const int esz = int8 ? 1 : 2, wq = int8 ? 1 : 2;
     // registers of the instance, as the compiler gives them within a few
@@ -294,6 +296,8 @@ double tile_time(const ConvParams& p, bool int8, const ConvChoice& c) {
            (r.overlap ? std::max(cu, block) : cu + block);
 }
 
+namespace {
+
 // Fastest estimated tile of a 3x3 conv; false (best as it was) where none applies.  With
 // a tile forced on the implicit GEMM that kernel is not among them (it runs,
 // with the forced tile, where no window kernel fits).
@@ -333,7 +337,7 @@ bool choose_conv3x3(const ConvParams& p, bool int8, ConvChoice& best) {
             // 32x32 MFMA: the widest tiles and the two-group blocks were the fastest at
             // a handful of shapes only, 8 waves of 4 subtiles lose up to 1.4x to others
             if (c.kind == 5 && (c.jn > 3 || c.ksw || (c.nw == 8 && c.jn * c.pw >= 4))) continue;
-            const double t = tile_time(p, int8, c);
+            const double t = conv_tile_time(p, int8, c);
             if (!e.found || t < best_t) {
                 best_t = t;
                 e.best = c;

@@ -29,6 +29,9 @@ namespace {
 // Parts of the amax pass: two blocks a CU, and no more words than a conv reads
 // (its waves read them all at their start).
 constexpr uint32_t kAmaxParts = 512;
+// Words of a pg16 command's parts (parts x groups): the conv's blocks read them
+// all at their start, 16 a thread at most.
+constexpr uint32_t kStripWords = 4096;
 constexpr uint32_t kMaxGroups = 32;  // 16-channel groups a per-tensor command takes (512 channels)
 
 struct DeviceScratch {
@@ -59,7 +62,7 @@ uint32_t* library_scratch(uint64_t words) {
 }  // namespace
 
 uint64_t int8_command_scratch_words(uint32_t in_channels) {
-    return std::max<uint64_t>(kAmaxParts, (in_channels + 15) / 16);
+    return std::max<uint64_t>(kStripWords, (in_channels + 15) / 16);
 }
 
 bool run_int8_command(const AexrtConv2DDesc& d, uint32_t algorithm, uint32_t flags, const AexrtHipTensorView& x,
@@ -108,10 +111,20 @@ bool run_int8_command(const AexrtConv2DDesc& d, uint32_t algorithm, uint32_t fla
     const __half* xd = static_cast<const __half*>(x.data);
     const int N = (int)d.batch, HW = (int)(d.in_h * d.in_w), C = (int)d.in_channels;
     if (pg16) {
-        if (!check_hip(launch_fill_u32(scratch, groups, 0u, stream), "conv2d_int8: clear amax") ||
-            !check_hip(launch_amax_strips_nhwc(xd, x.n_stride, x.c_stride, N, HW, C, scratch, stream),
-                       "conv2d_int8: amax pass"))
-            return false;
+        int parts = 0;
+        const int most = (int)(std::min<uint64_t>({scratch_words, kStripWords, kAmaxParts * groups}) / groups);
+        const hipError_t e =
+            launch_amax_strip_parts_nhwc(xd, x.n_stride, x.c_stride, N, HW, C, scratch, most, &parts, stream);
+        if (e == hipErrorNotSupported) {
+            // many channels of a large input: one copy of the strips, atomic updates
+            if (!check_hip(launch_fill_u32(scratch, groups, 0u, stream), "conv2d_int8: clear amax") ||
+                !check_hip(launch_amax_strips_nhwc(xd, x.n_stride, x.c_stride, N, HW, C, scratch, stream),
+                           "conv2d_int8: amax pass"))
+                return false;
+        } else {
+            if (!check_hip(e, "conv2d_int8: amax pass")) return false;
+            p.x_slots = SlotRef{scratch, (uint32_t)parts, groups};
+        }
     } else {
         int parts = 0;
         if (!check_hip(launch_amax_parts_nhwc(xd, x.n_stride, x.c_stride, N, HW, C, scratch, (int)kAmaxParts, &parts,

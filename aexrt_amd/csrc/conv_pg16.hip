@@ -4,22 +4,25 @@
 // The reference's pg16 conv (native/aexrt_d3d12_runtime.cpp:4770-4923) sums
 // the int8 products of one 16-channel group exactly in int32, scales each
 // group sum by amax[1 + g] / 127 into an fp32 accumulator, and finishes with
-// the oc weight scale, the bias and SiLU.  One v_mfma_i32_16x16x64_i8 covers
-// 64 input channels, i.e. four groups, and its sum would mix them.  Here the
-// A operand (weights) is made block-diagonal instead: of the 16 A rows, row
-// 4o + r carries output channel oc0 + 4o + j's weights of group r only (the
-// lanes of the three other lane groups read zero), so row 4o + r of the
-// product is the exact int32 sum of group r alone.  A lane of lane group grp
-// then holds the four group sums of one (output channel, position); four
-// MFMAs (j = 0..3) cover 16 output channels, and lane (grp, col) ends with
-// channels oc0 + 4 grp + j of position col -- the fragment layout of the
-// per-tensor kernels, so their epilogue and 8-byte NHWC stores are reused.
+// the oc weight scale, the bias and SiLU.  One v_mfma_i32_16x16x64_i8 takes 64
+// k, four times the 16 channels of a group, so its k holds one group at a time:
+// for a 3x3 conv the group's 16 channels of four taps (lane group grp loads tap
+// 4 i + grp of step i; three steps cover the nine taps, the last three k
+// quarters have zero weights), for a 1x1 conv the channels of four groups with
+// the weights of all but one zeroed (four products from one load of each
+// operand).  Rows are 16 output channels, columns 16 positions, so a lane ends
+// with channels oc0 + 4 grp + r of position col: the fragment layout of the
+// per-tensor kernels, whose epilogue and 8-byte NHWC stores are reused.
 //
 // The int32 group sums run over all taps of the kernel before the fp32
 // scaling (exact integers; the reference scales per tap for 3x3 and per 8
-// channels for 1x1, which differs only in fp32 rounding).  The MFMA work is
-// 4x that of the per-tensor kernel; at these shapes the kernels are bound by
-// memory latency and VALU, not by MFMA.
+// channels for 1x1, which differs only in fp32 rounding).
+//
+// Bound by the address lookups of its loads (16 bytes of 64 places each): with
+// one operand load for all lanes instead of one per lane group, 3 products per
+// group instead of 9 and JN subtiles on one input, 96 -> 48 at 27x35 x5 9.1 ->
+// 7.1 us, 512 -> 256 1x1 at 20x20 6.9 -> 5.8.  Two units in flight instead of one
+// were slower (8.7 us; the registers cost more than the latency).
 #include "conv_igemm.h"
 
 namespace aexrt {
@@ -39,32 +42,22 @@ constexpr int kPgMaxGroups = 256;  // in_channels <= 4096
 // LOADER kLoaderNhwc: fp16 NHWC view quantized here with 127/amax_g (the
 // reference's pack with per-group scales, RT:3330-3344); kLoaderPackedNc4: the
 // reference's packed NC/4HW4 int8 ((n * C/4 + icg) * H*W + pixel words).
-template <int KK, int LOADER>
+// A wave takes 16 positions and JN 16-channel subtiles.
+template <int KK, int LOADER, int JN>
 __global__ __launch_bounds__(kPgWaves * 64) void conv_int8_pg16_kernel(ConvParams p) {
+    constexpr int NB = KK == 9 ? 3 : 1;  // k steps of one unit: a group (3x3), four groups (1x1)
+    constexpr int R = JN * 16;
+    constexpr bool kPacked = LOADER == kLoaderPackedNc4;
+    __shared__ uint32_t l_max[kPgMaxGroups];
     __shared__ float l_gs[kPgMaxGroups];  // amax_g / 127
     __shared__ float l_qs[kPgMaxGroups];  // 127 / amax_g, 0 when amax_g is not > 0
-    __shared__ float l_bias[16], l_scale[16];
-    __shared__ uint32_t l_slots[1];
+    __shared__ float l_bias[R], l_scale[R];
+    __shared__ uint32_t l_slots[JN];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int col = lane & 15, grp = lane >> 4;
-    const int T = (p.C + 63) >> 6;  // 64-channel steps
     const int G = p.C >> 4;
-    for (int g = tid; g < 4 * T; g += kPgWaves * 64) {
-        uint32_t m = 0;
-        if (g < G)
-            for (uint32_t s = 0; s < p.x_slots.stripes; ++s) m = max(m, p.x_slots.p[s * p.x_slots.stride + g]);
-        const float a = u2f(m);
-        l_gs[g] = g < G ? a / 127.0f : 0.0f;
-        l_qs[g] = a > 0.0f ? 127.0f / a : 0.0f;
-    }
-    const int oc0 = blockIdx.y * 16;
-    if (tid < 16) {
-        const int oc = oc0 + tid;
-        l_bias[tid] = oc < p.OC ? p.bias[oc] : 0.0f;
-        l_scale[tid] = oc < p.OC ? p.w_scale[oc] : 0.0f;
-    }
-    if (tid == 0) l_slots[0] = 0u;
-    __syncthreads();
+    const int U = KK == 9 ? G : (p.C + 63) >> 6;
+    const int oc0 = blockIdx.y * R;
 
     const int m = (blockIdx.x * kPgWaves + wave) * 16 + col;
     const bool mok = m < p.M;
@@ -73,60 +66,121 @@ __global__ __launch_bounds__(kPgWaves * 64) void conv_int8_pg16_kernel(ConvParam
     const int pos = mm - n * p.OH * p.OW;
     const int oh = (int)fdiv((uint32_t)pos, p.fd_ow);
     const int ow = pos - oh * p.OW;
-    const int iy0 = oh * p.S - p.P, ix0 = ow * p.S - p.P;
     const uint32_t plane = (uint32_t)(p.H * p.W);
-
     const rsrc_t rx = make_rsrc(p.x, p.x_bytes);
     const rsrc_t rw = make_rsrc(p.w, (uint32_t)p.OCp * (uint32_t)p.Kp);
-    // element offset of (n, channel 0, pixel 0) in the input
-    const uint32_t xbase = LOADER == kLoaderPackedNc4 ? (uint32_t)n * (uint32_t)(p.C >> 2) * plane
-                                                      : (uint32_t)((int64_t)n * p.x_nstride);
-    // A row col = 4 o + r: output channel oc0 + 4 o + j, group r of the step;
-    // only lane group r loads it, every other lane reads zero
-    const int wo = col >> 2;
-    const bool wlane = (col & 3) == grp;
+    // byte offsets of this lane's pixel (channel 0) and weights (row col of the
+    // first subtile) of each k step; kOob and any channel offset on top of it
+    // stay past both buffers
+    uint32_t xo[NB], wo[NB];
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+        const int tap = KK == 9 ? 4 * i + grp : 0;
+        const int ky = tap / 3;
+        const int iy = oh * p.S - p.P + ky, ix = ow * p.S - p.P + (tap - 3 * ky);
+        const bool ok = mok && tap < KK && iy >= 0 && iy < p.H && ix >= 0 && ix < p.W;
+        const uint32_t pix = (uint32_t)(iy * p.W + ix);
+        if constexpr (kPacked) xo[i] = ok ? ((uint32_t)n * (uint32_t)(p.C >> 2) * plane + pix) * 4u : kOob;
+        else xo[i] = ok ? ((uint32_t)((int64_t)n * p.x_nstride) + pix * (uint32_t)p.x_cstride) * 2u : kOob;
+        wo[i] = tap < KK ? (uint32_t)(oc0 + col) * (uint32_t)p.Kp + (uint32_t)(tap * p.C) : kOob;
+    }
+    struct Unit {
+        v4i x[NB][kPacked ? 1 : 2], w[NB][JN];
+    };
+    // operands of unit u (past the last one: unused, inside the buffers' bounds checks)
+    auto load = [&](int u, Unit& q) {
+        const int c0 = KK == 9 ? 16 * u : 64 * u + 16 * grp;
+        const bool cok = KK == 9 || c0 < p.C;
+#pragma unroll
+        for (int i = 0; i < NB; ++i) {
+            if constexpr (kPacked) {
+#pragma unroll
+                for (int w = 0; w < 4; ++w)
+                    q.x[i][0][w] = __builtin_amdgcn_raw_buffer_load_b32(
+                        rx, cok ? xo[i] + (uint32_t)((c0 >> 2) + w) * plane * 4u : kOob, 0, 0);
+            } else {
+                q.x[i][0] = bload16(rx, cok ? xo[i] + (uint32_t)c0 * 2u : kOob);
+                q.x[i][1] = bload16(rx, cok ? xo[i] + (uint32_t)c0 * 2u + 16u : kOob);
+            }
+#pragma unroll
+            for (int j = 0; j < JN; ++j)
+                q.w[i][j] = bload16(rw, cok ? wo[i] + (uint32_t)(j * 16 * p.Kp + c0) : kOob);
+        }
+    };
+    Unit cur;
+    load(0, cur);
+
+    // group maxima: over the copies of the slot array (one thread per group and
+    // run of copies, then one LDS atomic each)
+    for (int g = tid; g < kPgMaxGroups; g += kPgWaves * 64) l_max[g] = 0u;
+    if (tid < R) {
+        const int oc = oc0 + tid;
+        l_bias[tid] = oc < p.OC ? p.bias[oc] : 0.0f;
+        l_scale[tid] = oc < p.OC ? p.w_scale[oc] : 0.0f;
+    }
+    if (tid < JN) l_slots[tid] = 0u;
+    __syncthreads();
+    {
+        const int row = (int)fdiv((uint32_t)tid, p.fd_ns), g = tid - row * G, rows = kPgWaves * 64 / G;
+        if (row < rows) {
+            uint32_t v = 0u;
+            for (uint32_t s = row; s < p.x_slots.stripes; s += rows) v = max(v, p.x_slots.p[s * p.x_slots.stride + g]);
+            if (v) atomicMax(&l_max[g], v);
+        }
+    }
+    __syncthreads();
+    for (int g = tid; g < ((G + 3) & ~3); g += kPgWaves * 64) {
+        const float a = u2f(l_max[g]);
+        l_gs[g] = g < G ? a / 127.0f : 0.0f;
+        l_qs[g] = a > 0.0f ? 127.0f / a : 0.0f;
+    }
+    __syncthreads();
 
     typedef float v4f_t __attribute__((ext_vector_type(4)));
-    v4f_t accf = {0.0f, 0.0f, 0.0f, 0.0f};  // channel oc0 + 4 grp + j
-    for (int t = 0; t < T; ++t) {
-        const int c0 = 64 * t + 16 * grp;  // this lane group's 16 channels
-        const bool cok = c0 < p.C;
-        v4i acc[4];
+    v4f_t accf[JN][1];  // channels oc0 + 16 j + 4 grp + r
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[j] = v4i{0, 0, 0, 0};
+    for (int j = 0; j < JN; ++j) accf[j][0] = v4f_t{0.0f, 0.0f, 0.0f, 0.0f};
+    auto quant = [&](const v4i (&x)[kPacked ? 1 : 2], float s) {
+        if constexpr (kPacked) return x[0];
+        const v2i q0 = quant8(x[0], s), q1 = quant8(x[kPacked ? 0 : 1], s);
+        return v4i{q0[0], q0[1], q1[0], q1[1]};
+    };
+    auto add = [&](int j, const v4i& acc, float s) {
 #pragma unroll
-        for (int tap = 0; tap < KK; ++tap) {
-            const int iy = iy0 + (KK == 9 ? tap / 3 : 0);
-            const int ix = ix0 + (KK == 9 ? tap % 3 : 0);
-            const bool ok = mok && cok && iy >= 0 && iy < p.H && ix >= 0 && ix < p.W;
-            const uint32_t pix = (uint32_t)(iy * p.W + ix);
-            v4i b;
-            if constexpr (LOADER == kLoaderPackedNc4) {
+        for (int r = 0; r < 4; ++r) accf[j][0][r] = __builtin_fmaf((float)acc[r], s, accf[j][0][r]);
+    };
+    auto multiply = [&](int u, const Unit& q) {
+        if constexpr (KK == 9) {
+            const float s = l_qs[u], gs = l_gs[u];
+            v4i acc[JN];
 #pragma unroll
-                for (int q = 0; q < 4; ++q)
-                    b[q] = __builtin_amdgcn_raw_buffer_load_b32(
-                        rx, ok ? (xbase + (uint32_t)((c0 >> 2) + q) * plane + pix) * 4u : kOob, 0, 0);
-            } else {
-                const uint32_t e = xbase + pix * (uint32_t)p.x_cstride + (uint32_t)c0;
-                const v4i lo = bload16(rx, ok ? e * 2u : kOob);
-                const v4i hi = bload16(rx, ok ? (e + 8u) * 2u : kOob);
-                const float s = l_qs[4 * t + grp];
-                const v2i q0 = quant8(lo, s), q1 = quant8(hi, s);
-                b = v4i{q0[0], q0[1], q1[0], q1[1]};
+            for (int j = 0; j < JN; ++j) acc[j] = v4i{0, 0, 0, 0};
+#pragma unroll
+            for (int i = 0; i < NB; ++i) {
+                const v4i b = quant(q.x[i], s);
+#pragma unroll
+                for (int j = 0; j < JN; ++j) acc[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(q.w[i][j], b, acc[j], 0, 0, 0);
             }
-            const uint32_t k = (uint32_t)(tap * p.C + c0);
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const uint32_t oc = (uint32_t)(oc0 + 4 * wo + j);
-                const v4i a = bload16(rw, wlane && cok ? oc * (uint32_t)p.Kp + k : kOob);
-                acc[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, acc[j], 0, 0, 0);
+            for (int j = 0; j < JN; ++j) add(j, acc[j], gs);
+        } else {
+            const v4i b = quant(q.x[0], l_qs[4 * u + grp]);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float gs = l_gs[4 * u + r];
+#pragma unroll
+                for (int j = 0; j < JN; ++j) {
+                    const v4i w = grp == r ? q.w[0][j] : v4i{0, 0, 0, 0};
+                    add(j, __builtin_amdgcn_mfma_i32_16x16x64_i8(w, b, v4i{0, 0, 0, 0}, 0, 0, 0), gs);
+                }
             }
         }
-        // acc[j][r] = int32 sum of group 4t + r for channel oc0 + 4 grp + j
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) accf[j] = __builtin_fmaf((float)acc[j][r], l_gs[4 * t + r], accf[j]);
+    };
+    for (int u = 0; u < U; ++u) {
+        Unit next;
+        load(u + 1, next);
+        multiply(u, cur);
+        cur = next;
     }
 
     const bool do_silu = (p.flags & kConvSilu) != 0;
@@ -136,18 +190,20 @@ __global__ __launch_bounds__(kPgWaves * 64) void conv_int8_pg16_kernel(ConvParam
         const rsrc_t ry = make_rsrc(p.y, p.y_bytes);
         const int ohw = p.OH * p.OW;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int lc = 4 * grp + j, oc = oc0 + lc;
-            float v = __builtin_fmaf(accf[j], l_scale[lc], l_bias[lc]);
-            if (do_silu) v = silu(v);
-            const bool ok = mok && oc < p.OC;
-            const uint32_t e = (uint32_t)((n * p.OC + oc) * ohw + pos);
-            if (out_f32)
-                __builtin_amdgcn_raw_buffer_store_b32(__float_as_int(v), ry, ok ? e * 4u : kOob, 0, 0);
-            else
-                __builtin_amdgcn_raw_buffer_store_b16(__half_as_short(__float2half(v)), ry, ok ? e * 2u : kOob, 0,
-                                                      0);
-        }
+        for (int j = 0; j < JN; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int lc = 16 * j + 4 * grp + r, oc = oc0 + lc;
+                float v = __builtin_fmaf(accf[j][0][r], l_scale[lc], l_bias[lc]);
+                if (do_silu) v = silu(v);
+                const bool ok = mok && oc < p.OC;
+                const uint32_t e = (uint32_t)((n * p.OC + oc) * ohw + pos);
+                if (out_f32)
+                    __builtin_amdgcn_raw_buffer_store_b32(__float_as_int(v), ry, ok ? e * 4u : kOob, 0, 0);
+                else
+                    __builtin_amdgcn_raw_buffer_store_b16(__half_as_short(__float2half(v)), ry, ok ? e * 2u : kOob, 0,
+                                                          0);
+            }
         return;
     }
     // NHWC view output: the per-tensor kernels' epilogue (scale, bias, SiLU,
@@ -155,17 +211,20 @@ __global__ __launch_bounds__(kPgWaves * 64) void conv_int8_pg16_kernel(ConvParam
     const rsrc_t ry = make_rsrc(p.y, p.y_bytes);
     const rsrc_t rr = make_rsrc(p.res, p.r_bytes);
     const rsrc_t racc = make_rsrc(nullptr, 0u);
+    const int jmax = min(JN, (p.OCp - oc0) >> 4);
     int yo[1], ro[1], mo[1];
     yo[0] = mok ? (int)((int64_t)n * p.y_nstride + (int64_t)pos * p.y_cstride) : -1;
     ro[0] = (int)((int64_t)n * p.r_nstride + (int64_t)pos * p.r_cstride);
     mo[0] = m;
-    v2i rv[1][1];
-    igemm::tile_residual<1, 1, igemm::kEpiAny>(p, rr, yo, ro, oc0, 1, grp, 1u, rv);
-    const v4f_t accs[1][1] = {{accf}};
-    float gmax[1] = {0.0f};
-    igemm::tile_store<true, 1, 1, igemm::kEpiAny>(p, accs, yo, mo, rv, oc0, 1, grp, 1u, l_bias, l_scale, gmax, ry,
-                                                  racc);
-    igemm::flush_slots<1>(p, gmax, oc0, 1, 1u, out_f32, l_slots);
+    constexpr uint32_t kAll = (1u << JN) - 1u;
+    v2i rv[JN][1];
+    igemm::tile_residual<JN, 1, igemm::kEpiAny>(p, rr, yo, ro, oc0, jmax, grp, kAll, rv);
+    float gmax[JN];
+#pragma unroll
+    for (int j = 0; j < JN; ++j) gmax[j] = 0.0f;
+    igemm::tile_store<true, JN, 1, igemm::kEpiAny>(p, accf, yo, mo, rv, oc0, jmax, grp, kAll, l_bias, l_scale, gmax,
+                                                   ry, racc);
+    igemm::flush_slots<JN>(p, gmax, oc0, jmax, kAll, out_f32, l_slots);
 }
 
 // a3: the reference's fused amax + pack (RT:4083-4149).  One block per
@@ -214,10 +273,29 @@ __global__ __launch_bounds__(kFusedThreads) void quant_fused_pg16_kernel(const T
     }
 }
 
+template <int KK, int LOADER, int JN>
+void launch_pg_tile(const ConvParams& p, hipStream_t stream) {
+    const dim3 grid((p.M + kPgWaves * 16 - 1) / (kPgWaves * 16), (p.OCp / 16 + JN - 1) / JN);
+    hipLaunchKernelGGL((conv_int8_pg16_kernel<KK, LOADER, JN>), grid, dim3(kPgWaves * 64), 0, stream, p);
+}
+
+// Blocks of 64 positions by 16 channels.
+int64_t pg_blocks(const ConvParams& p) {
+    return (int64_t)((p.M + kPgWaves * 16 - 1) / (kPgWaves * 16)) * (p.OCp / 16);
+}
+
+// More channel subtiles a wave read (and quantize) the input fewer times, once
+// the smaller grid still gives every CU more than one block: 1x1 128 -> 128 at
+// 40x40 x8 9.3 us with 1, 8.4 with 2, 7.7 with 4; 1x1 512 -> 256 at 20x20 (112
+// blocks) 5.8, 8.2, 10.3.  Four only where they leave no empty subtile (64 -> 80
+// at 40x40 x32: 12.4, 11.4, 12.1).
 template <int KK, int LOADER>
 void launch_pg(const ConvParams& p, hipStream_t stream) {
-    const dim3 grid((p.M + kPgWaves * 16 - 1) / (kPgWaves * 16), p.OCp / 16);
-    hipLaunchKernelGGL((conv_int8_pg16_kernel<KK, LOADER>), grid, dim3(kPgWaves * 64), 0, stream, p);
+    const int64_t blocks = pg_blocks(p);
+    const int ocj = p.OCp / 16;
+    if (ocj % 4 == 0 && blocks / 4 >= 384) launch_pg_tile<KK, LOADER, 4>(p, stream);
+    else if (ocj > 1 && blocks / 2 >= 384) launch_pg_tile<KK, LOADER, 2>(p, stream);
+    else launch_pg_tile<KK, LOADER, 1>(p, stream);
 }
 
 uint64_t span_nhwc(int N, int64_t nstride, int32_t cstride, int HW, int C, int esz) {
@@ -270,6 +348,20 @@ hipError_t launch_conv_int8_pg16(const ConvParams& p0, hipStream_t stream) {
         }
         p.fd_ohw = make_fastdiv((uint32_t)HWo);
         p.fd_ow = make_fastdiv((uint32_t)p.OW);
+        p.fd_ns = make_fastdiv((uint32_t)(p.C / 16));
+        // the window kernel quantizes an input element once instead of up to nine
+        // times per 16 channels, and reads weights from LDS; its longer start and
+        // its barrier per group cost more on short grids of few groups.  us, this
+        // kernel and the window kernel: 128 -> 128 at 40x40 x16 73.5, 29.4; 64 -> 64 at
+        // 40x40 x8 (800 blocks) 16.7, 8.5; 256 -> 256 at 20x20 (112) 16.0, 13.7; 96 -> 48
+        // at 27x35 x5 (222) 7.1, 9.2; 48 -> 144 at 33x17 x3 (243) 4.8, 6.4; 320 -> 96 at
+        // 7x7 (6) 13.8, 19.6
+        const int64_t blocks = pg_blocks(p);
+        if (!packed && !nchw_out && p.KH == 3 && (blocks >= 400 || (blocks >= 64 && p.C >= 128))) {
+            const hipError_t e = launch_conv_halo_pg16(p, stream);
+            if (e == hipSuccess) continue;
+            if (e != hipErrorNotSupported) return e;
+        }
         if (p.KH == 1) {
             if (packed) launch_pg<1, kLoaderPackedNc4>(p, stream);
             else launch_pg<1, kLoaderNhwc>(p, stream);

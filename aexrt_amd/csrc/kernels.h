@@ -204,6 +204,11 @@ int enumerate_halo_choices(const ConvParams& p, bool int8, ConvChoice* out, int 
 hipError_t launch_conv_halo(const ConvParams& p, bool int8, int epi, hipStream_t stream);
 // False while set_conv3x3_halo turns the halo-tile kernel off or forces its tile.
 bool halo_mode_auto();
+// pg16 form of it (a scale per 16 input channels) on one batch slice, NHWC in
+// and out, tile chosen here; hipErrorNotSupported where it does not apply.
+hipError_t launch_conv_halo_pg16(const ConvParams& p, hipStream_t stream);
+// Estimated microseconds of a 3x3 conv with tile c (kinds 1, 2, 5).
+double conv_tile_time(const ConvParams& p, bool int8, const ConvChoice& c);
 // Halo kernel selection for 3x3 convs: mode 0 automatic, 1 never (implicit
 // GEMM only), 2 forced tile (jn oc subtiles, pw position subtiles per wave,
 // tr x tc output positions per tile, cc channels per chunk; a 3x3 conv the
@@ -311,6 +316,11 @@ hipError_t launch_amax_slots_nhwc(const __half* x, int64_t nstride, int32_t cstr
 // nothing to clear.  C % 16 == 0.
 hipError_t launch_amax_parts_nhwc(const __half* x, int64_t nstride, int32_t cstride, int N, int HW, int C,
                                   uint32_t* parts, int max_parts, int* count, hipStream_t stream);
+// The pg16 strip maxima in parts: parts[b * C/16 + s] = max|x| of strip s in
+// share b (*count <= max_parts shares); nothing to clear.  hipErrorNotSupported
+// where max_parts is too few for the tensor.  C % 16 == 0.
+hipError_t launch_amax_strip_parts_nhwc(const __half* x, int64_t nstride, int32_t cstride, int N, int HW, int C,
+                                        uint32_t* parts, int max_parts, int* count, hipStream_t stream);
 // Strips of the reference's amax buffer over an NHWC fp16 view: max|x| of
 // image n, group g folded into slots[(n * C/16 + g) / N], i.e. memory strip
 // (n*C + 16g) / (16N) of the NCHW layout (slots[s] = the reference's
