@@ -35,10 +35,13 @@ class ConvDesc(Structure):
 
     @classmethod
     def from_params(cls, params) -> "ConvDesc":
-        vals = [int(v) for v in params]
+        vals = params if isinstance(params, (list, tuple)) else list(params)
         if len(vals) != 16:
             raise ValueError("conv params must have 16 values")
-        return cls(*vals)
+        try:
+            return cls(*vals)
+        except TypeError:  # not all Python ints
+            return cls(*(int(v) for v in vals))
 
     def as_list(self) -> list[int]:
         return [int(getattr(self, f[0])) for f in self._fields_]
