@@ -168,8 +168,9 @@ def yolo_decode_nms_topk(out, *, classes: int, layout: int = 1, has_objectness: 
     if a.dtype != torch.float32 or not a.is_contiguous():
         raise ValueError("output0 must be a contiguous fp32 tensor")
     channels, anchors = (a.shape[1], a.shape[0]) if layout == 2 else (a.shape[0], a.shape[1])
-    dets = torch.zeros((max_detections, 6), dtype=torch.float32, device=a.device)
-    count = torch.zeros(1, dtype=torch.int32, device=a.device)
+    # the kernel writes the count and every row below it: nothing to clear (two launches)
+    dets = torch.empty((max_detections, 6), dtype=torch.float32, device=a.device)
+    count = torch.empty(1, dtype=torch.int32, device=a.device)
     check(_lib.lib().aexrt_hip_yolo_decode_nms_topk(
         a.data_ptr(), layout, anchors, channels, classes, int(has_objectness), float(conf), float(iou),
         max_candidates, max_detections, dets.data_ptr(), count.data_ptr(), _stream(stream)), "yolo_decode_nms_topk")
@@ -187,8 +188,9 @@ def yolo_dfl_decode_nms_topk(head, levels, *, classes: int, layout: int = 1, con
         raise ValueError("head must be a contiguous fp32 tensor")
     hw = (ctypes.c_uint32 * (2 * len(levels)))(*[int(v) for h, w, _ in levels for v in (h, w)])
     st = (ctypes.c_float * len(levels))(*[float(s) for _, _, s in levels])
-    dets = torch.zeros((max_detections, 6), dtype=torch.float32, device=a.device)
-    count = torch.zeros(1, dtype=torch.int32, device=a.device)
+    # the kernel writes the count and every row below it: nothing to clear (two launches)
+    dets = torch.empty((max_detections, 6), dtype=torch.float32, device=a.device)
+    count = torch.empty(1, dtype=torch.int32, device=a.device)
     check(_lib.lib().aexrt_hip_yolo_dfl_decode_nms_topk(
         a.data_ptr(), layout, len(levels), hw, st, classes, float(conf), float(iou), max_candidates, max_detections,
         dets.data_ptr(), count.data_ptr(), _stream(stream)), "yolo_dfl_decode_nms_topk")
