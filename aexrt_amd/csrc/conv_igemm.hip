@@ -5,7 +5,6 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
-#include <vector>
 
 #include "conv_igemm.h"
 
@@ -345,8 +344,8 @@ bool choose_conv3x3(const ConvParams& p, bool int8, ConvChoice& best) {
     for (int v : key) h = (h ^ (uint32_t)v) * 16777619u;
     Entry& e = memo[(h ^ (h >> 16)) % kEntries];
     if (std::memcmp(e.key, key, sizeof(key)) != 0) {
-        thread_local std::vector<ConvChoice> all(kMaxConvChoices);
-        const int n = enumerate_conv_choices(p, int8, all.data(), kMaxConvChoices);
+        ConvChoice all[kMaxConvChoices];
+        const int n = enumerate_conv_choices(p, int8, all, kMaxConvChoices);
         const ConvTile usual_tile = choose_conv_tile(p.M, p.OC, p.Kp);
         double best_t = 0.0;
         e.found = false;
