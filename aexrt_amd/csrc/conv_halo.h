@@ -582,6 +582,16 @@ hipError_t halo_launch_family(const HaloParams& h, int jn, int pw, int np, int n
     AEXRT_HALO_CASE(1, 1, 8) AEXRT_HALO_CASE(1, 2, 8) AEXRT_HALO_CASE(1, 4, 8)
     AEXRT_HALO_CASE(2, 1, 8) AEXRT_HALO_CASE(2, 2, 8) AEXRT_HALO_CASE(2, 4, 8)
     AEXRT_HALO_CASE(4, 1, 8) AEXRT_HALO_CASE(4, 2, 8) AEXRT_HALO_CASE(4, 4, 8)
+    // one position subtile a wave: windows of 5 and 6 pieces a thread on their own, as
+    // every round is bounds checks, a load and four registers of each iteration
+    // (int8 64 -> 128 from 160x160 x32, 5 rounds instead of 8: 67.2 -> 63.8 us; 112 ->
+    // 32 at 150x150 x7 24.1 -> 20.7; no conv of 270 random ones over 2 % slower).  2
+    // and 3 instead of 4 free registers for more resident blocks, whose shorter runs
+    // of tiles cost a whole network 0.6 %
+#define AEXRT_HALO_CASES(J) \
+    AEXRT_HALO_CASE(J, 1, 5) AEXRT_HALO_CASE(J, 1, 6)
+    AEXRT_HALO_CASES(1) AEXRT_HALO_CASES(2) AEXRT_HALO_CASES(4)
+#undef AEXRT_HALO_CASES
 #undef AEXRT_HALO_CASE
     // 8 waves: the block's weights shared by twice the positions
 #define AEXRT_HALO_CASE8(J, P, N) \
@@ -589,6 +599,10 @@ hipError_t halo_launch_family(const HaloParams& h, int jn, int pw, int np, int n
     AEXRT_HALO_CASE8(1, 1, 4) AEXRT_HALO_CASE8(1, 2, 4) AEXRT_HALO_CASE8(2, 1, 4) AEXRT_HALO_CASE8(2, 2, 4)
     AEXRT_HALO_CASE8(4, 1, 4) AEXRT_HALO_CASE8(4, 2, 4) AEXRT_HALO_CASE8(1, 1, 8) AEXRT_HALO_CASE8(1, 2, 8)
     AEXRT_HALO_CASE8(2, 1, 8) AEXRT_HALO_CASE8(2, 2, 8) AEXRT_HALO_CASE8(4, 1, 8) AEXRT_HALO_CASE8(4, 2, 8)
+#define AEXRT_HALO_CASES8(J) \
+    AEXRT_HALO_CASE8(J, 1, 5) AEXRT_HALO_CASE8(J, 1, 6)
+    AEXRT_HALO_CASES8(1) AEXRT_HALO_CASES8(2) AEXRT_HALO_CASES8(4)
+#undef AEXRT_HALO_CASES8
     // every output channel of an 80-channel conv in one block (weights up to
     // 128 KB, one block per CU)
     if constexpr (!INT8) {

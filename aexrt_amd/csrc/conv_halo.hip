@@ -356,12 +356,16 @@ hipError_t launch_conv_halo(const ConvParams& p, bool int8, int epi, hipStream_t
         }
         // a forced tile that does not fit this conv is an error, not a
         // silent fallback (tests rely on the tile being used)
-        t.np = 4;
-        if (!halo_geometry(h, t, int8)) {
-            t.np = 8;
-            HaloParams h8 = h;
-            if (!halo_geometry(h8, t, int8)) return hipErrorInvalidValue;
+        // (the NCHW loader and tiles of several position subtiles have instances of 4 and 8 pieces)
+        bool fits = false;
+        for (int np : {4, 5, 6, 8}) {
+            if (np != 4 && np != 8 && (t.pw != 1 || t.jn > 4 || p.loader == kLoaderNchwF32)) continue;
+            t.np = np;
+            HaloParams hh = h;
+            fits = halo_geometry(hh, t, int8);
+            if (fits) break;
         }
+        if (!fits) return hipErrorInvalidValue;
     } else if (p.loader != kLoaderNchwF32 || !choose_nchw_tile(h, t)) {
         return hipErrorNotSupported;  // NHWC tiles are chosen by the caller
     }

@@ -203,7 +203,7 @@ namespace {
 // tiles of 4 waves by a clock count, implicit GEMM only where no halo tile fits)
 // took 1.15x: 4 waves leave a CU half empty where the weights fill the LDS, and
 // it never took the 32x32-MFMA kernel.  Examples, us before and after: int8
-// 64 -> 128 channels at 80x80 from 160x160 x32 81.8 -> 69.7, 256 at 40x40 x2 17.9
+// 64 -> 128 channels at 80x80 from 160x160 x32 81.8 -> 63.8, 256 at 40x40 x2 17.9
 // -> 11.4, 512 at 20x20 38.7 -> 14.4; fp16 128 at 80x80 x4 29.5 -> 22.6, 256 -> 64
 // at 20x20 x8 17.1 -> 10.8.
 struct TileRates {
